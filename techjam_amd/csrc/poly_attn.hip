@@ -82,6 +82,7 @@ constexpr size_t kPerHead = kTokImg + 2 * kTokImgBytes;
 constexpr int kRing = 3;                        // quad-state stages in flight
 constexpr int kRingStage = 2 * PD * PD * 2;     // one stage: rows of two i, [2][64 v][64 j] fp16
 constexpr int kStageBytes = kRing * kRingStage;
+static_assert(kPerHead < (size_t(1) << 31), "workspace offsets of one head fit a buffer resource");
 static_assert(kStageBytes >= 4 * 64 * LP * 2, "diagonal / update tiles must fit the ring area");
 constexpr int kSmemBytes = kStageBytes;
 
@@ -101,6 +102,18 @@ struct PolyArgs {
   char* ws;
   int M;                // B * H
 };
+
+// One direct global->LDS copy of a wave: 16 bytes per lane from byte offset
+// soff + voff of the head's workspace to lds + 16 * lane. A buffer load, not
+// global_load_lds: the compiler counts that one as a FLAT access, and while
+// one is in flight turns every wait for an LDS read into lgkmcnt(0), so that
+// reads issued ahead of the MFMAs they feed would be waited for at once.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t head_rsrc(const char* ws) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(ws), (short)0, (int)kPerHead, kBufferFlags);
+}
+__device__ __forceinline__ void copy_to_lds(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+}
 
 __device__ __forceinline__ float4_t ld4(const float* p) { return *reinterpret_cast<const float4_t*>(p); }
 
@@ -200,12 +213,9 @@ struct TokTile {
   }
 };
 
-__device__ __forceinline__ half8_t mul8(half8_t x, half_t s) {
-  half8_t r;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = x[j] * s;
-  return r;
-}
+// x * s as four packed multiplies. (Element by element the compiler emits
+// eight scalar multiplies and four packs.)
+__device__ __forceinline__ half8_t mul8(half8_t x, half_t s) { return x * half8_t{s, s, s, s, s, s, s, s}; }
 
 // ---------------------------------------------------------------------------
 // Apply role: rows [row0, row0 + 256) of the chunk; each wave owns RB = 2
@@ -222,7 +232,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
   auto kb = reinterpret_cast<half_t(*)[64][LP]>(smem);                  // diag: [2][64][LP]
   auto vt = reinterpret_cast<half_t(*)[64][LP]>(smem + 2 * 64 * LP * 2);  // diag: [2][64][LP]
 
-  const int tid = threadIdx.x, w = tid / kWave, lane = tid % kWave, hl = lane / 32, ln = lane % 32;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave, hl = lane / 32, ln = lane % 32;
   const int qw0 = row0 + WROWS * w;
 
   // a = fp16(q * rs); B operand slots (hl, j) <-> dim 16*ks + 8*hl + j.
@@ -267,7 +277,8 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
     return __builtin_bit_cast(half2_t, ((p >> 2) & 1) ? r[1] : r[0]);
   };
 
-  const half_t* qshadow = reinterpret_cast<const half_t*>(ws + kQuadShadow) + size_t(slot) * PD * PD * PD;
+  const __amdgpu_buffer_rsrc_t rws = head_rsrc(ws);
+  const uint32_t qshadow = uint32_t(kQuadShadow) + slot * (PD * PD * PD * 2);
   // The fp16 quad shadow of one i is piece-major, [8 q][64 v][8 j]: piece q
   // holds columns j = 8q .. 8q + 7 of every row v (1 KiB contiguous per q).
   // It streams through a ring of kRing LDS stages by direct global->LDS
@@ -307,9 +318,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
       const int k = w + 4 * it;
       const int gp = k / (2 * np), rem = k % (2 * np);
       const int q = 2 * ib + (rem >> 1), ii = rem & 1;
-      const half_t* src = qshadow + (size_t(2 * (p0 + gp) + ii) * 8 + q) * (PD * 8) + lane * 8;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(base + k * 1024), 16, 0, 0);
+      copy_to_lds(rws, base + k * 1024, lane * 16, qshadow + ((2 * (p0 + gp) + ii) * 8 + q) * (PD * 8 * 2));
     }
   };
 
@@ -504,9 +513,14 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 
 // The token images of the chunks this launch folds in stream through a ring
 // of three LDS stages by direct global->LDS copies issued two tiles ahead (no
-// registers held). body(bT, vT) runs on every 64-token tile (b^T and v^T, 64
-// dim rows of 128 bytes with XOR-placed 16-byte pieces, see img_piece);
-// chunk_end(j) after the last tile of the launch's j-th chunk, once the
+// registers held). A 64-token tile is four MFMA k-steps; load(bT, vT, ks)
+// reads one step's operands (b^T and v^T, 64 dim rows of 128 bytes with
+// XOR-placed 16-byte pieces, see img_piece) and mma(ops) consumes them. The
+// operands of step ks + 1 -- across the tile boundary too -- are read before
+// step ks's MFMAs, so the LDS latency is under them: with one or two waves
+// per SIMD nothing else hides it (a tile took ~3000 cycles against 1024 of
+// MFMA when each step read its own operands first). chunk_end(j) runs after
+// the last tile of the launch's j-th chunk, once the
 // workgroup has passed that tile's barrier: its global stores then complete
 // under the next tile instead of holding up the wait for the copies (issued
 // before them) that the barrier needs. The stages are
@@ -524,13 +538,14 @@ __device__ __forceinline__ half8_t img_piece(const half_t* base, int row, int pc
   return *reinterpret_cast<const half8_t*>(reinterpret_cast<const char*>(base) + row * 128 + 16 * (pc ^ ((row >> 1) & 7)));
 }
 
-template <typename Body, typename ChunkEnd>
-__device__ __forceinline__ void stream_image(const char* img, int n_chunk, char* smem, Body&& body,
-                                             ChunkEnd&& chunk_end) {
+template <typename Load, typename Mma, typename ChunkEnd>
+__device__ __forceinline__ void stream_image(const char* ws, uint32_t img, int n_chunk, char* smem, Load&& load,
+                                             Mma&& mma, ChunkEnd&& chunk_end) {
   constexpr int kTiles = PC / 64;
   TokRing& ring = *reinterpret_cast<TokRing*>(smem);
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int n = n_chunk * kTiles;
+  const __amdgpu_buffer_rsrc_t rws = head_rsrc(ws);
   auto stage_ptr = [&](auto st) -> char* {
     if constexpr (decltype(st)::value == 0) return ring.s0;
     else if constexpr (decltype(st)::value == 1) return ring.s1;
@@ -539,12 +554,10 @@ __device__ __forceinline__ void stream_image(const char* img, int n_chunk, char*
   // Copy instruction `it` of wave w moves 1 KiB slot 4 it + w of the tile.
   auto issue = [&](int t, auto st) {
     char* base = stage_ptr(st);
-    const char* src = img + size_t(t) * kTileImg;
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int slot = 4 * it + w;
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + slot * 1024 + lane * 16),
-                                       (__attribute__((address_space(3))) void*)(base + slot * 1024), 16, 0, 0);
+      copy_to_lds(rws, base + slot * 1024, lane * 16, img + t * kTileImg + slot * 1024);
     }
   };
   // Tile t + 1 (this wave's four copies) must have landed before the barrier;
@@ -556,18 +569,38 @@ __device__ __forceinline__ void stream_image(const char* img, int n_chunk, char*
     else __builtin_amdgcn_s_waitcnt(0x0070);            // vmcnt(0) lgkmcnt(0)
     lds_barrier();
   };
+  using Ops = decltype(load((const half_t*)nullptr, (const half_t*)nullptr, 0));
+  Ops ops[2];
+  auto load_ks = [&](char* base, int ks) {
+    return load(reinterpret_cast<const half_t*>(base), reinterpret_cast<const half_t*>(base + PD * 128), ks);
+  };
   auto step = [&](int t, auto st) {
     constexpr int sv = decltype(st)::value;
     if (t + 2 < n) issue(t + 2, std::integral_constant<int, (sv + 2) % 3>{});
-    const char* base = stage_ptr(st);
-    body(reinterpret_cast<const half_t*>(base), reinterpret_cast<const half_t*>(base + PD * 128));
-    wait_next(t);
+    char* base = stage_ptr(st);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) {
+        ops[(ks + 1) & 1] = load_ks(base, ks + 1);
+      } else {
+        // This wave's last operands of tile t are in registers (lgkmcnt(0)),
+        // so past the barrier the tile's stage may be refilled.
+        wait_next(t);
+        if (t + 1 < n) ops[0] = load_ks(stage_ptr(std::integral_constant<int, (sv + 1) % 3>{}), 0);
+      }
+      // This step's operands are there; the next step's may stay in flight.
+      if (ks < 3 || t + 1 < n) __builtin_amdgcn_s_waitcnt(0xC07F | (sizeof(Ops) / 16) << 8);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(ops[ks & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if ((t + 1) % kTiles == 0) chunk_end(t / kTiles);
   };
   if (n == 0) return;
   issue(0, std::integral_constant<int, 0>{});
   if (n > 1) issue(1, std::integral_constant<int, 1>{});
   wait_next(-1);
+  ops[0] = load_ks(ring.s0, 0);
   for (int t = 0; t < n; t += 3) {
     step(t, std::integral_constant<int, 0>{});
     if (t + 1 < n) step(t + 1, std::integral_constant<int, 1>{});
@@ -633,6 +666,9 @@ __device__ __forceinline__ void quad_update_body(const PolyArgs& a, char* ws, in
   update_range(a, c0, c1);
   if (c0 >= c1) return;
   constexpr int NJ = 2 - JB0;
+  struct Ops {
+    half8_t bj[NJ], vv[2], bi[NI];
+  };
   const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
   float* img = reinterpret_cast<float*>(ws + kQuadImg);
   // acc[ii][jj][vb] = D[j][v] block (jb = JB0 + jj) of S_{i0+ii}. The fp32
@@ -645,31 +681,31 @@ __device__ __forceinline__ void quad_update_body(const PolyArgs& a, char* ws, in
 #pragma unroll
       for (int vb = 0; vb < 2; ++vb) load_img(img + ((size_t(i0 + ii) * 2 + JB0 + jj) * 2 + vb) * 1024, acc[ii][jj][vb]);
 
-  const char* tok = ws + kTokImg + size_t(a.launch & 1) * kTokImgBytes;
+  const uint32_t tok = uint32_t(kTokImg) + (a.launch & 1) * uint32_t(kTokImgBytes);
   stream_image(
-      tok, c1 - c0, smem,
-      [&](const half_t* bT, const half_t* vT) {
+      ws, tok, c1 - c0, smem,
+      [&](const half_t* bT, const half_t* vT, int ks) {
+        const int pc = 2 * ks + hl;  // tokens 16 ks + 8 hl .. +7 of the tile
+        Ops o;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const int pc = 2 * ks + hl;  // tokens 16 ks + 8 hl .. +7 of the tile
-          half8_t bj[NJ], vv[2];
+        for (int jj = 0; jj < NJ; ++jj) o.bj[jj] = img_piece(bT, 32 * (JB0 + jj) + ln, pc);
 #pragma unroll
-          for (int jj = 0; jj < NJ; ++jj) bj[jj] = img_piece(bT, 32 * (JB0 + jj) + ln, pc);
+        for (int x = 0; x < 2; ++x) o.vv[x] = img_piece(vT, 32 * x + ln, pc);
 #pragma unroll
-          for (int x = 0; x < 2; ++x) vv[x] = img_piece(vT, 32 * x + ln, pc);
+        for (int ii = 0; ii < NI; ++ii) o.bi[ii] = img_piece(bT, i0 + ii, pc);
+        return o;
+      },
+      [&](const Ops& o) {
 #pragma unroll
-          for (int ii = 0; ii < NI; ++ii) {
-            const half8_t bi = img_piece(bT, i0 + ii, pc);
+        for (int ii = 0; ii < NI; ++ii)
 #pragma unroll
-            for (int jj = 0; jj < NJ; ++jj) {
-              half8_t phi;
+          for (int jj = 0; jj < NJ; ++jj) {
+            half8_t phi;
 #pragma unroll
-              for (int j = 0; j < 8; ++j) phi[j] = bj[jj][j] * bi[j];
+            for (int j = 0; j < 8; ++j) phi[j] = o.bj[jj][j] * o.bi[ii][j];
 #pragma unroll
-              for (int vb = 0; vb < 2; ++vb) acc[ii][jj][vb] = mfma32(phi, vv[vb], acc[ii][jj][vb]);
-            }
+            for (int vb = 0; vb < 2; ++vb) acc[ii][jj][vb] = mfma32(phi, o.vv[vb], acc[ii][jj][vb]);
           }
-        }
       },
       [&](int j) {
         // fp16 shadow of state_{c+1} for the applies of the next launch: only
@@ -704,99 +740,98 @@ __device__ __forceinline__ void quad_update_role(const PolyArgs& a, char* ws, in
   else quad_update_body<4, 1>(a, ws, 32 + 16 * (ug - 4) + 4 * w, smem);
 }
 
+// One wave each: S_lin[j][v] = sum_t b_tj v_tv, G[i][j] = sum_t b_ti b_tj (as
+// 2x2 accumulator blocks each), z[d] = sum_t b_td and S_const[d] = sum_t v_td
+// (lane = dim; four running sums, so the adds do not wait on one another).
+template <bool GRAM>
+__device__ __forceinline__ void small_mfma_wave(char* ws, uint32_t tok, int c0, int c1, char* smem) {
+  struct Ops {
+    half8_t r[2], c[2];
+  };
+  const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
+  float* img = reinterpret_cast<float*>(ws + (GRAM ? kGramImg : kLinImg));
+  float16_t acc[2][2];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) load_img(img + (rb * 2 + cb) * 1024, acc[rb][cb]);
+  stream_image(
+      ws, tok, c1 - c0, smem,
+      [&](const half_t* bT, const half_t* vT, int ks) {
+        const int pc = 2 * ks + hl;
+        Ops o;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          o.r[x] = img_piece(bT, 32 * x + ln, pc);
+          if constexpr (!GRAM) o.c[x] = img_piece(vT, 32 * x + ln, pc);
+        }
+        return o;
+      },
+      [&](const Ops& o) {
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = mfma32(o.r[rb], GRAM ? o.r[cb] : o.c[cb], acc[rb][cb]);
+      },
+      [&](int j) {
+        const int nxt = (c0 + j + 1) % NSLOT;  // S_lin as [v][j]; G is symmetric
+        half_t* sh = reinterpret_cast<half_t*>(ws + (GRAM ? kGramShadow : kLinShadow)) + size_t(nxt) * PD * PD;
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) store_shadow_t(sh, acc[rb][cb], rb, cb);
+      });
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) store_img(img + (rb * 2 + cb) * 1024, acc[rb][cb]);
+}
+
+template <bool CONST>
+__device__ __forceinline__ void small_sum_wave(char* ws, uint32_t tok, int c0, int c1, char* smem) {
+  struct Ops {
+    half8_t x[2];
+  };
+  const int lane = threadIdx.x % kWave;
+  float* master = reinterpret_cast<float*>(ws + kZsMaster) + (CONST ? 64 : 0);
+  float total = master[lane];
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
+  stream_image(
+      ws, tok, c1 - c0, smem,
+      [&](const half_t* bT, const half_t* vT, int ks) {
+        Ops o;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) o.x[x] = img_piece(CONST ? vT : bT, lane, 2 * ks + x);
+        return o;
+      },
+      [&](const Ops& o) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          part[j & 1] += (float)o.x[0][j];
+          part[2 + (j & 1)] += (float)o.x[1][j];
+        }
+      },
+      [&](int j) {
+        total += (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) part[x] = 0.f;
+        reinterpret_cast<float*>(ws + kZsShadow)[(c0 + j + 1) % NSLOT * 128 + (CONST ? 64 : 0) + lane] = total;
+      });
+  master[lane] = total;
+}
+
 __device__ __forceinline__ void small_update_role(const PolyArgs& a, char* ws, char* smem) {
   int c0, c1;
   update_range(a, c0, c1);
   if (c0 >= c1) return;
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
-  float* lin_img = reinterpret_cast<float*>(ws + kLinImg);
-  float* gram_img = reinterpret_cast<float*>(ws + kGramImg);
-  float* zs = reinterpret_cast<float*>(ws + kZsMaster);
-  float16_t acc[2][2];
-  if (w < 2) {
-    float* img = w == 0 ? lin_img : gram_img;
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) load_img(img + (rb * 2 + cb) * 1024, acc[rb][cb]);
-  }
-  float z = 0.f, cs = 0.f;
-  if (w == 2) {
-    z = zs[lane];
-    cs = zs[64 + lane];
-  }
-  float zsum = 0.f, csum = 0.f;
-  const char* tok = ws + kTokImg + size_t(a.launch & 1) * kTokImgBytes;
-  stream_image(
-      tok, c1 - c0, smem,
-      [&](const half_t* bT, const half_t* vT) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          const int pc = 2 * ks + hl;
-          if (w == 0) {  // S_lin[j][v] = sum_t b_tj v_tv
-#pragma unroll
-            for (int jb = 0; jb < 2; ++jb) {
-              const half8_t bj = img_piece(bT, 32 * jb + ln, pc);
-#pragma unroll
-              for (int vb = 0; vb < 2; ++vb) acc[jb][vb] = mfma32(bj, img_piece(vT, 32 * vb + ln, pc), acc[jb][vb]);
-            }
-          } else if (w == 1) {  // G[i][j] = sum_t b_ti b_tj
-#pragma unroll
-            for (int ib = 0; ib < 2; ++ib) {
-              const half8_t bi = img_piece(bT, 32 * ib + ln, pc);
-#pragma unroll
-              for (int jb = 0; jb < 2; ++jb) acc[ib][jb] = mfma32(bi, img_piece(bT, 32 * jb + ln, pc), acc[ib][jb]);
-            }
-          } else if (w == 2) {  // z[d] and S_const[d]: lane = dim, 16 tokens per step
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-              const half8_t bx = img_piece(bT, lane, 2 * ks + half);
-              const half8_t vx = img_piece(vT, lane, 2 * ks + half);
-#pragma unroll
-              for (int j = 0; j < 8; ++j) {
-                zsum += (float)bx[j];
-                csum += (float)vx[j];
-              }
-            }
-          }
-        }
-      },
-      [&](int j) {
-        const int nxt = (c0 + j + 1) % NSLOT;
-        if (w == 0) {
-          half_t* sh = reinterpret_cast<half_t*>(ws + kLinShadow) + size_t(nxt) * PD * PD;  // [v][j]
-#pragma unroll
-          for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-            for (int vb = 0; vb < 2; ++vb) store_shadow_t(sh, acc[jb][vb], jb, vb);
-        } else if (w == 1) {
-          half_t* sh = reinterpret_cast<half_t*>(ws + kGramShadow) + size_t(nxt) * PD * PD;  // symmetric
-#pragma unroll
-          for (int ib = 0; ib < 2; ++ib)
-#pragma unroll
-            for (int jb = 0; jb < 2; ++jb) store_shadow_t(sh, acc[ib][jb], ib, jb);
-        } else if (w == 2) {
-          z += zsum;
-          cs += csum;
-          zsum = csum = 0.f;
-          float* zsh = reinterpret_cast<float*>(ws + kZsShadow) + nxt * 128;
-          zsh[lane] = z;
-          zsh[64 + lane] = cs;
-        }
-      });
-  if (w == 0) {
-#pragma unroll
-    for (int jb = 0; jb < 2; ++jb)
-#pragma unroll
-      for (int vb = 0; vb < 2; ++vb) store_img(lin_img + (jb * 2 + vb) * 1024, acc[jb][vb]);
-  } else if (w == 1) {
-#pragma unroll
-    for (int ib = 0; ib < 2; ++ib)
-#pragma unroll
-      for (int jb = 0; jb < 2; ++jb) store_img(gram_img + (ib * 2 + jb) * 1024, acc[ib][jb]);
-  } else if (w == 2) {
-    zs[lane] = z;
-    zs[64 + lane] = cs;
+  const uint32_t tok = uint32_t(kTokImg) + (a.launch & 1) * uint32_t(kTokImgBytes);
+  // The waves take different code (a scalar branch) but the same barriers,
+  // one per tile.
+  switch (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) {
+    case 0: small_mfma_wave<false>(ws, tok, c0, c1, smem); break;
+    case 1: small_mfma_wave<true>(ws, tok, c0, c1, smem); break;
+    case 2: small_sum_wave<false>(ws, tok, c0, c1, smem); break;
+    default: small_sum_wave<true>(ws, tok, c0, c1, smem); break;
   }
 }
 

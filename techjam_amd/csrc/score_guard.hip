@@ -15,7 +15,7 @@
 // and component e of every piece is one MFMA k-step (any assignment of dims
 // to k-steps works as long as both operands share it). So nothing is staged
 // in LDS and every load of a tile is in flight at once; what bounds a
-// workgroup is the latency of one row gather plus 4096 MFMA cycles per wave
+// workgroup is the latency of one row gather plus 2048 MFMA cycles per wave
 // and key block at head_dim 64. Measured at 16 heads of 100 000 fp16 tokens:
 // 56 -> 25 us (before: 64x64 blocks staged through LDS by 4 waves, 4x4
 // FMA tiles, eight key blocks one after another).
