@@ -11,8 +11,8 @@
 //   S_quad[(i,j), v] += sum_t b_ti b_tj v_tv,  S_lin[j, v] += sum_t b_tj v_tv,
 //   G[i, j] += sum_t b_ti b_tj,  z[j] += sum_t b_tj,  S_const[v] += sum_t v_tv.
 //
-// Launches advance KG = 16 chunks at a time; in launch L every head owns 55
-// workgroups with four roles:
+// Launches advance one window of KG = 16 chunks at a time; in launch L every
+// head owns workgroups with five roles (P, 1 or 2, is the split below):
 //   * apply (2 per chunk, 256 rows each, for the KG chunks whose start
 //     states the previous launch produced): quadratic term as
 //       y^T = sum_i S_i^T (a_i * a^T)  (S_i = rows (i, .) of S_quad),
@@ -20,27 +20,35 @@
 //     registers -- phi2(a) never exists in memory; linear and denominator terms
 //     as three more small GEMMs; the exact diagonal block like the exact
 //     kernel (S^T = b a^T in registers, no max subtraction).
-//   * quad update (6 per head): S_i += (b_i * b)^T v over the tokens of
-//     chunks [KG L, KG L + KG), accumulated straight into MFMA accumulators
-//     that hold the fp32 master in its register image (the master's memory
-//     layout IS the accumulator layout, so loading and storing it is straight
-//     16-byte copies, once per launch). After each chunk it writes the fp16
-//     shadow of the state the apply of the next chunk reads.
-//   * small-state update (1 per head): S_lin, G, z, S_const, likewise.
-//   * token images (KG per head): b = k*sqrt(scale) and v of the chunks the
-//     next launch folds in, converted once to fp16 tiles laid out as the
-//     update roles' LDS image, which those roles then stream with direct
+//   * state update (6 quad + 1 small per head and part): S_i += (b_i * b)^T v
+//     over the tokens of the part's KG / P chunks of window L, accumulated
+//     straight into MFMA accumulators that hold the fp32 state in its register
+//     image (the state's memory layout IS the accumulator layout, so loading
+//     and storing it is straight 16-byte copies); S_lin, G, z, S_const
+//     likewise. A part starts from the state at the window's start plus the
+//     sums of the parts before it; the last part stores the next window's
+//     start. After each chunk it writes the fp16 shadow of the state the apply
+//     of the next chunk reads.
+//   * part sums (7 per head for each part of window L + 1 but the last, when
+//     P > 1): the same folding from zero, without shadows, into an fp32 sum.
+//   * token images (KG per head): b = k*sqrt(scale) and v of a later window
+//     (L + 1; L + 2 when P > 1), converted once to fp16 tiles laid out as
+//     the update roles' LDS image, which those roles then stream with direct
 //     global->LDS copies.
 // State c (before chunk c) lives in shadow slot c % (2 KG): a launch reads
 // the slots of states KG L - KG + 1 .. KG L and writes those of KG L + 1 ..
 // KG L + KG, so applies and updates of one launch never touch the same slot.
-// More chunks per launch load and store each master less often and need
+// Window starts, part sums and images are buffered by window, so that no role
+// of a launch writes what another one reads.
+// More chunks per launch load and store each state less often and need
 // fewer launches (the polynomial call on 64 heads of 65536 tokens: 4 -> 8
 // chunks 5.8-6.1 -> 5.4-5.5 ms; the extreme step with 8 -> 16 chunks
-// 8.99-9.02 -> 8.78-8.83 ms, 10.2 MiB more workspace per head), at the
-// price of a longer update chain per launch when few heads share the GPU
-// (16 heads of 100 000 tokens: 2.39-2.40 -> 2.42 ms).
-// Heads whose guard flag is 0 exit at once (the exact kernel covers them).
+// 8.99-9.02 -> 8.78-8.83 ms, 10.2 MiB more workspace per head).
+//
+// Parts. A window is a chain of KG * 8 token tiles for each update workgroup
+// (~0.8 us a tile), while seven of them per head leave the chip idle for a
+// few heads. P parts fold KG / P chunks each, all at once, at the price of
+// folding all but one part twice; see parts_for().
 #include <type_traits>
 
 #include "tj_common.h"
@@ -56,26 +64,45 @@ constexpr int NUPD = 6;        // quad-update workgroups per head (4 for i < 32,
 constexpr int KG = 16;         // chunks per launch (update sub-chunks, apply groups)
 constexpr int NSLOT = 2 * KG;  // shadow slots: state_c lives in slot c % NSLOT
 constexpr int NCONV = KG;      // token-image workgroups per head (one chunk each)
-constexpr int NROLE = KG * NAPPLY + NUPD + 1 + NCONV;
+constexpr int NSTATE = NUPD + 1;  // state-update workgroups per head and part
+constexpr int PMAX = 2;        // most parts of a window
+constexpr int NIMG = 4;        // token-image buffers: window w in buffer w % NIMG
 constexpr int LP = 72;         // padded LDS row of 64 halves (144 bytes)
 constexpr int kBufferFlags = 0x00020000;  // raw (untyped) buffer resource word 3 on gfx950
 
+// One state (byte offsets): S_quad without the j < 32 blocks of i >= 32, which
+// nothing reads (S_ij = S_ji), in accumulator images of [64 lanes][16] fp32.
+constexpr uint32_t kImg = 64 * 16 * 4;
+constexpr uint32_t kStQuad = 0;                        // [i < 32][2 jb][2 vb], then [i >= 32][2 vb] (jb = 1)
+constexpr uint32_t kStLin = (32 * 4 + 32 * 2) * kImg;  // [2 jb][2 vb]
+constexpr uint32_t kStGram = kStLin + 4 * kImg;        // [2 ib][2 jb]
+constexpr uint32_t kStZs = kStGram + 4 * kImg;         // fp32 z[64], S_const[64]
+constexpr uint32_t kStateBytes = kStZs + 128 * 4;
+__host__ __device__ constexpr uint32_t quad_img(int i, int jb, int vb) {
+  return kStQuad + (i < 32 ? (i * 2 + jb) * 2 + vb : 128 + (i - 32) * 2 + vb) * kImg;
+}
+// fp16 quad shadow of one state, piece-major: for each i the pieces q = j / 8
+// >= 2 (i / 16) that the apply reads, [q][64 v][8 j] (1 KiB each).
+__host__ __device__ constexpr uint32_t quad_shadow(int i) {
+  const int ib = i >> 4;
+  return 1024u * (16 * (9 * ib - ib * ib) + (i & 15) * (8 - 2 * ib));
+}
+constexpr uint32_t kShadowBytes = quad_shadow(64);
+static_assert(quad_shadow(16) == 1024 * 128 && quad_shadow(32) == 1024 * 224 && kShadowBytes == 1024 * 320, "pieces");
+
 // Workspace of one head (byte offsets).
-constexpr size_t kQuadImg = 0;                                   // fp32 [64 i][2 jb][2 vb][64 lanes][16]
-constexpr size_t kQuadImgBytes = size_t(PD) * 4 * 64 * 16 * 4;  // 1 MiB
-constexpr size_t kLinImg = kQuadImg + kQuadImgBytes;             // fp32 [2 jb][2 vb][64][16]
-constexpr size_t kGramImg = kLinImg + 4 * 64 * 16 * 4;           // fp32 [2 ib][2 jb][64][16]
-constexpr size_t kZsMaster = kGramImg + 4 * 64 * 16 * 4;         // fp32 z[64], S_const[64]
-constexpr size_t kQuadShadow = kZsMaster + 128 * 4;              // fp16 [NSLOT][64 i][8 q][64 v][8 j]
-constexpr size_t kLinShadow = kQuadShadow + NSLOT * size_t(PD) * PD * PD * 2;  // fp16 [NSLOT][64 v][64 j]
-constexpr size_t kGramShadow = kLinShadow + NSLOT * PD * PD * 2;  // fp16 [NSLOT][64][64] (symmetric)
-constexpr size_t kZsShadow = kGramShadow + NSLOT * PD * PD * 2;   // fp32 [NSLOT][128]
-// Token images: the k (scaled) and v tiles the update roles of a launch fold
-// in, written once by the previous launch as fp16 LDS images (see TokTile).
-constexpr int kTileImg = 2 * PD * 64 * 2;                          // [b^T | v^T] of 64 tokens
-constexpr size_t kTokImgBytes = size_t(KG) * (PC / 64) * kTileImg;  // one launch: 2 MiB
-constexpr size_t kTokImg = (kZsShadow + NSLOT * 128 * 4 + 255) & ~size_t(255);  // [2][kTokImgBytes]
-constexpr size_t kPerHead = kTokImg + 2 * kTokImgBytes;
+constexpr uint32_t kStart = 0;                                  // window starts [2][kStateBytes]
+constexpr uint32_t kPart = kStart + 2 * kStateBytes;             // part sums [2][PMAX - 1][kStateBytes]
+constexpr uint32_t kQuadShadow = kPart + 2 * (PMAX - 1) * kStateBytes;  // fp16 [NSLOT][kShadowBytes]
+constexpr uint32_t kLinShadow = kQuadShadow + NSLOT * kShadowBytes;     // fp16 [NSLOT][64 v][64 j]
+constexpr uint32_t kGramShadow = kLinShadow + NSLOT * PD * PD * 2;      // fp16 [NSLOT][64][64] (symmetric)
+constexpr uint32_t kZsShadow = kGramShadow + NSLOT * PD * PD * 2;       // fp32 [NSLOT][128]
+// Token images: the k (scaled) and v tiles of a window, as fp16 LDS images
+// (see TokTile).
+constexpr int kTileImg = 2 * PD * 64 * 2;                            // [b^T | v^T] of 64 tokens
+constexpr uint32_t kTokImgBytes = uint32_t(KG) * (PC / 64) * kTileImg;  // one window: 2 MiB
+constexpr uint32_t kTokImg = (kZsShadow + NSLOT * 128 * 4 + 255) & ~255u;  // [NIMG][kTokImgBytes]
+constexpr size_t kPerHead = size_t(kTokImg) + NIMG * kTokImgBytes;
 
 // LDS: apply = quad-state ring (49152) or diagonal tiles (36864);
 //      updates = two transposed token tiles, double buffered (36864).
@@ -95,6 +122,7 @@ struct PolyArgs {
   int H, S;
   float rs;             // sqrt(scale)
   int launch;           // launch index L: applies chunks (KG (L-1), KG L], updates [KG L, KG L + KG)
+  int parts;            // P
   int n_chunks;
   int prefix_end;       // rows below are left to the exact kernel
   const float* coeffs;  // [M][3]
@@ -261,6 +289,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     float dl = 0.f;
+    if (c > 0)
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -278,21 +307,19 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
   };
 
   const __amdgpu_buffer_rsrc_t rws = head_rsrc(ws);
-  const uint32_t qshadow = uint32_t(kQuadShadow) + slot * (PD * PD * PD * 2);
-  // The fp16 quad shadow of one i is piece-major, [8 q][64 v][8 j]: piece q
-  // holds columns j = 8q .. 8q + 7 of every row v (1 KiB contiguous per q).
-  // It streams through a ring of kRing LDS stages by direct global->LDS
-  // copies two stages ahead of the MFMAs (no registers held). Pair p
-  // (i = 2p, 2p + 1) only reads the pieces q >= 2 ib, ib = p >> 3 (S is
-  // symmetric, see the step), np = 8 - 2 ib of them per row, so a stage holds
-  // G pairs (G = 1, 1, 2, 4 for ib = 0 .. 3, at most 16 KiB) as
-  // [gp][q - 2 ib][ii][64 v] 16-byte pieces (1 KiB per (gp, q, ii)), filled
-  // by 2 G np copy instructions (k = 2 (gp np + q - 2 ib) + ii; wave w issues
-  // k = w, w + 4, ...): 37.5 % fewer bytes than whole rows, 22 stages instead
-  // of 32, and 16 lanes reading one piece column of 16 consecutive rows touch
-  // 256 contiguous bytes. The stages are distinct members addressed with
-  // compile-time indices, so the compiler can tell the copies into one stage
-  // from reads of another and does not wait for every copy in flight.
+  const uint32_t qshadow = kQuadShadow + slot * kShadowBytes;
+  // The quad shadow streams through a ring of kRing LDS stages by direct
+  // global->LDS copies two stages ahead of the MFMAs (no registers held).
+  // Pair p (i = 2p, 2p + 1) has the pieces q >= 2 ib, ib = p >> 3 (S is
+  // symmetric, see the step), np = 8 - 2 ib of them per i, so a stage holds
+  // G pairs (G = 1, 1, 2, 4 for ib = 0 .. 3, at most 16 KiB), contiguous in
+  // the shadow: [2 gp + ii][q - 2 ib][64 v] 16-byte pieces, filled by 2 G np
+  // copy instructions of 1 KiB (wave w issues k = w, w + 4, ...): 37.5 % fewer
+  // bytes than whole rows, 22 stages instead of 32, and 16 lanes reading one
+  // piece column of 16 consecutive rows touch 256 contiguous bytes. The stages
+  // are distinct members addressed with compile-time indices, so the compiler
+  // can tell the copies into one stage from reads of another and does not wait
+  // for every copy in flight.
   struct Ring {
     char s0[kRingStage];
     char s1[kRingStage];
@@ -316,9 +343,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 #pragma unroll
     for (int it = 0; it < G * np / 2; ++it) {
       const int k = w + 4 * it;
-      const int gp = k / (2 * np), rem = k % (2 * np);
-      const int q = 2 * ib + (rem >> 1), ii = rem & 1;
-      copy_to_lds(rws, base + k * 1024, lane * 16, qshadow + ((2 * (p0 + gp) + ii) * 8 + q) * (PD * 8 * 2));
+      copy_to_lds(rws, base + k * 1024, lane * 16, qshadow + quad_shadow(2 * p0) + k * 1024);
     }
   };
 
@@ -353,7 +378,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
       for (int ii = 0; ii < 2; ++ii) {
 #pragma unroll
         for (int ks = ib; ks < 4; ++ks) {
-          const int k = 2 * (gp * np + 2 * ks + hl - 2 * ib) + ii;
+          const int k = (2 * gp + ii) * np + 2 * ks + hl - 2 * ib;
           half8_t sa[2];
 #pragma unroll
           for (int vb = 0; vb < 2; ++vb) sa[vb] = *reinterpret_cast<const half8_t*>(base + k * 1024 + (32 * vb + ln) * 16);
@@ -378,11 +403,13 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
     }
     lds_barrier();
   };
-  issue(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-  issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
-  __builtin_amdgcn_s_waitcnt(0x0074);  // stage 0 landed (stage 1: four copies in flight)
-  lds_barrier();
-  static_for<0, kSteps>(step);
+  if (c > 0) {  // the state before chunk 0 is zero, and no launch wrote it
+    issue(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
+    issue(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+    __builtin_amdgcn_s_waitcnt(0x0074);  // stage 0 landed (stage 1: four copies in flight)
+    lds_barrier();
+    static_for<0, kSteps>(step);
+  }
 
   // Linear numerator term S_lin^T a^T and the quadratic denominator G a^T
   // (operands straight from the L2-resident shadows). G's rows are read in
@@ -400,7 +427,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
   // One 32-row block of S_lin^T (output block blk = v block) and of G at a time,
   // each fragment feeding both query blocks.
 #pragma unroll
-  for (int blk = 0; blk < 2; ++blk) {
+  for (int blk = 0; blk < (c > 0 ? 2 : 0); ++blk) {
     half8_t la[4], ga[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
@@ -494,7 +521,7 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int v0 = 32 * vb + 8 * g + 4 * hl;
-        const float4_t sc = ld4(zs + 64 + v0);
+        const float4_t sc = c > 0 ? ld4(zs + 64 + v0) : float4_t{0.f, 0.f, 0.f, 0.f};
         float y[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = (c0 * sc[e] + accq[rb][vb][4 * g + e]) * inv;
@@ -608,17 +635,18 @@ __device__ __forceinline__ void stream_image(const char* ws, uint32_t img, int n
   }
 }
 
-__device__ __forceinline__ void load_img(const float* img, float16_t& acc) {
+__device__ __forceinline__ void add_img(const char* img, float16_t& acc) {
   const int lane = threadIdx.x % kWave;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float4_t x = ld4(img + lane * 16 + 4 * q);
+    const float4_t x = ld4(reinterpret_cast<const float*>(img) + lane * 16 + 4 * q);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[4 * q + e] = x[e];
+    for (int e = 0; e < 4; ++e) acc[4 * q + e] += x[e];
   }
 }
 
-__device__ __forceinline__ void store_img(float* img, const float16_t& acc) {
+__device__ __forceinline__ void store_img(char* dst, const float16_t& acc) {
+  float* img = reinterpret_cast<float*>(dst);
   const int lane = threadIdx.x % kWave;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
@@ -637,53 +665,90 @@ __device__ __forceinline__ void store_shadow_t(half_t* dst, const float16_t& acc
   }
 }
 
-// The same block written into the piece-major quad shadow of S_i,
-// [8 q][64 v][8 j] (q = j / 8), as the apply's ring reads it, from row group
-// g0 on (g0 = 2 skips j = 32 rb .. 32 rb + 15).
-__device__ __forceinline__ void store_quad_shadow(half_t* dst, const float16_t& acc, int rb, int cb, int g0) {
+// The same block written into the piece-major quad shadow of S_i (dst, whose
+// first piece is q0), [q - q0][64 v][8 j], as the apply's ring reads it; row
+// groups before piece q0 are skipped (j = 32 rb .. 32 rb + 15 for odd i / 16).
+__device__ __forceinline__ void store_quad_shadow(half_t* dst, const float16_t& acc, int rb, int cb, int q0) {
   const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    if (g < g0) continue;
     const int j = 32 * rb + 8 * g + 4 * hl;  // four consecutive j, one piece
-    *reinterpret_cast<half4_t*>(dst + ((j >> 3) * 64 + 32 * cb + ln) * 8 + (j & 7)) =
+    if (4 * rb + g < q0) continue;
+    *reinterpret_cast<half4_t*>(dst + ((4 * rb + g - q0) * 64 + 32 * cb + ln) * 8 + (j & 7)) =
         half4_t{(half_t)acc[4 * g], (half_t)acc[4 * g + 1], (half_t)acc[4 * g + 2], (half_t)acc[4 * g + 3]};
   }
 }
 
-// Chunks whose states this launch folds in: [c0, c1) (the final chunk's
-// update is never needed).
-__device__ __forceinline__ void update_range(const PolyArgs& a, int& c0, int& c1) {
-  c0 = KG * a.launch;
-  c1 = min(c0 + KG, a.n_chunks - 1);
+// What one state workgroup folds: chunks [c0, c1) of window c0 / KG onto the
+// states listed, and where the result goes.
+struct Fold {
+  int c0, c1;
+  uint32_t tok;         // its token images (workspace offset)
+  uint32_t start;       // the window's start state, 0xffffffff for none (zero)
+  uint32_t part;        // part sums added to it: n_part states from here
+  int n_part;
+  uint32_t dst;         // the folded state, 0xffffffff if nobody reads it
+  bool shadow;          // write the fp16 shadow after every chunk
+
+  // f(state) for every state the fold starts from.
+  template <typename F>
+  __device__ __forceinline__ void sources(const char* ws, F&& f) const {
+    if (start != 0xffffffffu) f(ws + start);
+    for (int i = 0; i < n_part; ++i) f(ws + part + i * kStateBytes);
+  }
+};
+
+// Update of part p of window L, or (sum) the part's sum for window L + 1. The
+// final chunk's update is never needed; false when nothing is left to fold.
+__device__ __forceinline__ bool make_fold(const PolyArgs& a, int p, bool sum, Fold& f) {
+  const int win = a.launch + (sum ? 1 : 0), len = KG / a.parts;
+  const int last = a.n_chunks - 1;
+  if (win < 0) return false;
+  f.c0 = KG * win + p * len;
+  f.c1 = min(f.c0 + len, last);
+  // A sum is wanted only if the part after it has chunks.
+  if (f.c0 >= f.c1 || (sum && f.c0 + len >= last)) return false;
+  const uint32_t parts = kPart + (win & 1) * (PMAX - 1) * kStateBytes;
+  f.tok = kTokImg + uint32_t(win % NIMG) * kTokImgBytes + uint32_t(p * len) * (PC / 64) * kTileImg;
+  f.start = sum || win == 0 ? 0xffffffffu : kStart + (win & 1) * kStateBytes;
+  f.part = parts;
+  f.n_part = sum ? 0 : p;
+  f.dst = sum ? parts + p * kStateBytes
+              : (p == a.parts - 1 && KG * (win + 1) < last ? kStart + ((win + 1) & 1) * kStateBytes : 0xffffffffu);
+  f.shadow = !sum;
+  return true;
 }
 
 // NI i-slices per wave, j-blocks JB0..1 (the apply never reads j < 32 for
 // i >= 32: S is symmetric).
 template <int NI, int JB0>
-__device__ __forceinline__ void quad_update_body(const PolyArgs& a, char* ws, int i0, char* smem) {
-  int c0, c1;
-  update_range(a, c0, c1);
-  if (c0 >= c1) return;
+__device__ __forceinline__ void quad_update_body(const Fold& f, char* ws, int i0, char* smem) {
   constexpr int NJ = 2 - JB0;
   struct Ops {
     half8_t bj[NJ], vv[2], bi[NI];
   };
   const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
-  float* img = reinterpret_cast<float*>(ws + kQuadImg);
   // acc[ii][jj][vb] = D[j][v] block (jb = JB0 + jj) of S_{i0+ii}. The fp32
-  // master stays in these registers across the launch's chunks.
+  // state stays in these registers across the fold's chunks.
   float16_t acc[NI][NJ][2];
+  auto blocks = [&](auto&& g) {
 #pragma unroll
-  for (int ii = 0; ii < NI; ++ii)
+    for (int ii = 0; ii < NI; ++ii)
 #pragma unroll
-    for (int jj = 0; jj < NJ; ++jj)
+      for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
-      for (int vb = 0; vb < 2; ++vb) load_img(img + ((size_t(i0 + ii) * 2 + JB0 + jj) * 2 + vb) * 1024, acc[ii][jj][vb]);
+        for (int vb = 0; vb < 2; ++vb) g(i0 + ii, JB0 + jj, vb, acc[ii][jj][vb]);
+  };
+  blocks([](int, int, int, float16_t& x) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = 0.f;
+  });
+  f.sources(ws, [&](const char* st) {
+    blocks([&](int i, int jb, int vb, float16_t& x) { add_img(st + quad_img(i, jb, vb), x); });
+  });
 
-  const uint32_t tok = uint32_t(kTokImg) + (a.launch & 1) * uint32_t(kTokImgBytes);
   stream_image(
-      ws, tok, c1 - c0, smem,
+      ws, f.tok, f.c1 - f.c0, smem,
       [&](const half_t* bT, const half_t* vT, int ks) {
         const int pc = 2 * ks + hl;  // tokens 16 ks + 8 hl .. +7 of the tile
         Ops o;
@@ -709,54 +774,47 @@ __device__ __forceinline__ void quad_update_body(const PolyArgs& a, char* ws, in
       },
       [&](int j) {
         // fp16 shadow of state_{c+1} for the applies of the next launch: only
-        // the pieces the apply reads. For i in 16..31 and 48..63 it skips the
-        // 16 columns j below i's own 16-block (S is symmetric), which are the
-        // first half of this wave's first j-block.
-        const int c = c0 + j;
-        half_t* sh = reinterpret_cast<half_t*>(ws + kQuadShadow) + size_t((c + 1) % NSLOT) * PD * PD * PD;
-#pragma unroll
-        for (int ii = 0; ii < NI; ++ii)
-#pragma unroll
-          for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-            for (int vb = 0; vb < 2; ++vb)
-              store_quad_shadow(sh + size_t(i0 + ii) * PD * PD, acc[ii][jj][vb], JB0 + jj, vb,
-                                jj == 0 && ((i0 + ii) & 16) ? 2 : 0);
+        // the pieces the apply reads.
+        if (!f.shadow) return;
+        char* sh = ws + kQuadShadow + uint32_t((f.c0 + j + 1) % NSLOT) * kShadowBytes;
+        blocks([&](int i, int jb, int vb, const float16_t& x) {
+          store_quad_shadow(reinterpret_cast<half_t*>(sh + quad_shadow(i)), x, jb, vb, 2 * (i >> 4));
+        });
       });
-#pragma unroll
-  for (int ii = 0; ii < NI; ++ii)
-#pragma unroll
-    for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-      for (int vb = 0; vb < 2; ++vb) store_img(img + ((size_t(i0 + ii) * 2 + JB0 + jj) * 2 + vb) * 1024, acc[ii][jj][vb]);
+  if (f.dst != 0xffffffffu)
+    blocks([&](int i, int jb, int vb, const float16_t& x) { store_img(ws + f.dst + quad_img(i, jb, vb), x); });
 }
 
 // Quad-update workgroups 0..3: i < 32, two slices per wave, both j-blocks;
 // workgroups 4..5: i >= 32, four slices per wave, j >= 32 only -- the same
 // MFMA count per wave.
-__device__ __forceinline__ void quad_update_role(const PolyArgs& a, char* ws, int ug, char* smem) {
-  const int w = threadIdx.x / kWave;
-  if (ug < 4) quad_update_body<2, 0>(a, ws, 8 * ug + 2 * w, smem);
-  else quad_update_body<4, 1>(a, ws, 32 + 16 * (ug - 4) + 4 * w, smem);
+__device__ __forceinline__ void quad_update_role(const Fold& f, char* ws, int ug, char* smem) {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  if (ug < 4) quad_update_body<2, 0>(f, ws, 8 * ug + 2 * w, smem);
+  else quad_update_body<4, 1>(f, ws, 32 + 16 * (ug - 4) + 4 * w, smem);
 }
 
 // One wave each: S_lin[j][v] = sum_t b_tj v_tv, G[i][j] = sum_t b_ti b_tj (as
 // 2x2 accumulator blocks each), z[d] = sum_t b_td and S_const[d] = sum_t v_td
 // (lane = dim; four running sums, so the adds do not wait on one another).
 template <bool GRAM>
-__device__ __forceinline__ void small_mfma_wave(char* ws, uint32_t tok, int c0, int c1, char* smem) {
+__device__ __forceinline__ void small_mfma_wave(const Fold& f, char* ws, char* smem) {
   struct Ops {
     half8_t r[2], c[2];
   };
   const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
-  float* img = reinterpret_cast<float*>(ws + (GRAM ? kGramImg : kLinImg));
+  constexpr uint32_t img = GRAM ? kStGram : kStLin;
   float16_t acc[2][2];
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+  for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb) load_img(img + (rb * 2 + cb) * 1024, acc[rb][cb]);
+    for (int r = 0; r < 16; ++r) acc[b >> 1][b & 1][r] = 0.f;
+  f.sources(ws, [&](const char* st) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) add_img(st + img + b * kImg, acc[b >> 1][b & 1]);
+  });
   stream_image(
-      ws, tok, c1 - c0, smem,
+      ws, f.tok, f.c1 - f.c0, smem,
       [&](const half_t* bT, const half_t* vT, int ks) {
         const int pc = 2 * ks + hl;
         Ops o;
@@ -774,30 +832,31 @@ __device__ __forceinline__ void small_mfma_wave(char* ws, uint32_t tok, int c0, 
           for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = mfma32(o.r[rb], GRAM ? o.r[cb] : o.c[cb], acc[rb][cb]);
       },
       [&](int j) {
-        const int nxt = (c0 + j + 1) % NSLOT;  // S_lin as [v][j]; G is symmetric
+        if (!f.shadow) return;
+        const int nxt = (f.c0 + j + 1) % NSLOT;  // S_lin as [v][j]; G is symmetric
         half_t* sh = reinterpret_cast<half_t*>(ws + (GRAM ? kGramShadow : kLinShadow)) + size_t(nxt) * PD * PD;
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
           for (int cb = 0; cb < 2; ++cb) store_shadow_t(sh, acc[rb][cb], rb, cb);
       });
+  if (f.dst == 0xffffffffu) return;
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) store_img(img + (rb * 2 + cb) * 1024, acc[rb][cb]);
+  for (int b = 0; b < 4; ++b) store_img(ws + f.dst + img + b * kImg, acc[b >> 1][b & 1]);
 }
 
 template <bool CONST>
-__device__ __forceinline__ void small_sum_wave(char* ws, uint32_t tok, int c0, int c1, char* smem) {
+__device__ __forceinline__ void small_sum_wave(const Fold& f, char* ws, char* smem) {
   struct Ops {
     half8_t x[2];
   };
   const int lane = threadIdx.x % kWave;
-  float* master = reinterpret_cast<float*>(ws + kZsMaster) + (CONST ? 64 : 0);
-  float total = master[lane];
+  constexpr uint32_t at = kStZs + (CONST ? 64 * 4 : 0);
+  float total = 0.f;
+  f.sources(ws, [&](const char* st) { total += reinterpret_cast<const float*>(st + at)[lane]; });
   float part[4] = {0.f, 0.f, 0.f, 0.f};
   stream_image(
-      ws, tok, c1 - c0, smem,
+      ws, f.tok, f.c1 - f.c0, smem,
       [&](const half_t* bT, const half_t* vT, int ks) {
         Ops o;
 #pragma unroll
@@ -815,35 +874,35 @@ __device__ __forceinline__ void small_sum_wave(char* ws, uint32_t tok, int c0, i
         total += (part[0] + part[1]) + (part[2] + part[3]);
 #pragma unroll
         for (int x = 0; x < 4; ++x) part[x] = 0.f;
-        reinterpret_cast<float*>(ws + kZsShadow)[(c0 + j + 1) % NSLOT * 128 + (CONST ? 64 : 0) + lane] = total;
+        if (f.shadow)
+          reinterpret_cast<float*>(ws + kZsShadow)[(f.c0 + j + 1) % NSLOT * 128 + (CONST ? 64 : 0) + lane] = total;
       });
-  master[lane] = total;
+  if (f.dst != 0xffffffffu) reinterpret_cast<float*>(ws + f.dst + at)[lane] = total;
 }
 
-__device__ __forceinline__ void small_update_role(const PolyArgs& a, char* ws, char* smem) {
-  int c0, c1;
-  update_range(a, c0, c1);
-  if (c0 >= c1) return;
-  const uint32_t tok = uint32_t(kTokImg) + (a.launch & 1) * uint32_t(kTokImgBytes);
+__device__ __forceinline__ void small_update_role(const Fold& f, char* ws, char* smem) {
   // The waves take different code (a scalar branch) but the same barriers,
   // one per tile.
   switch (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave)) {
-    case 0: small_mfma_wave<false>(ws, tok, c0, c1, smem); break;
-    case 1: small_mfma_wave<true>(ws, tok, c0, c1, smem); break;
-    case 2: small_sum_wave<false>(ws, tok, c0, c1, smem); break;
-    default: small_sum_wave<true>(ws, tok, c0, c1, smem); break;
+    case 0: small_mfma_wave<false>(f, ws, smem); break;
+    case 1: small_mfma_wave<true>(f, ws, smem); break;
+    case 2: small_sum_wave<false>(f, ws, smem); break;
+    default: small_sum_wave<true>(f, ws, smem); break;
   }
 }
 
-// Token images of the chunks the next launch folds in, [KG (L+1), KG (L+1) +
-// KG): chunk j of them by workgroup j, eight 64-token tiles, loads of the next
-// tile in flight while the current one is stored.
+// Windows between the images a launch writes and its own: the updates read
+// window L, the part sums window L + 1.
+__host__ __device__ constexpr int image_lag(int parts) { return parts > 1 ? 2 : 1; }
+
+// Token images of chunk j of a later window: eight 64-token tiles, loads of
+// the next tile in flight while the current one is stored.
 template <typename T>
 __device__ void image_role(const PolyArgs& a, char* ws, int b, int h, int j) {
-  const int cn = KG * (a.launch + 1);
-  const int c = cn + j;
-  if (c >= min(cn + KG, a.n_chunks - 1)) return;
-  char* dst = ws + kTokImg + size_t((a.launch + 1) & 1) * kTokImgBytes + size_t(j) * (PC / 64) * kTileImg;
+  const int win = a.launch + image_lag(a.parts);
+  const int c = KG * win + j;
+  if (c >= a.n_chunks - 1) return;
+  char* dst = ws + kTokImg + uint32_t(win % NIMG) * kTokImgBytes + uint32_t(j) * (PC / 64) * kTileImg;
   const int tid = threadIdx.x;
   TokTile<T> x0, x1;
   x0.init(a, b, h, tid);
@@ -858,76 +917,62 @@ __device__ void image_role(const PolyArgs& a, char* ws, int b, int h, int j) {
   }
 }
 
-// Roles of one head in launch L: NUPD quad-update workgroups and one
-// small-state update folding in chunks [KG L, KG L + KG); KG * NAPPLY apply
-// workgroups (chunk KG (L-1) + 1 + j / NAPPLY, row block j % NAPPLY; launch 0
-// applies chunk 0 only); NCONV workgroups writing the token images of the
-// chunks launch L + 1 folds in. Launch -1 writes only the images for launch 0.
+// Roles of one head in launch L, longest first: NSTATE workgroups for each of
+// the P update parts of window L and of the P - 1 part sums of window L + 1;
+// KG * NAPPLY apply workgroups (chunk KG (L-1) + 1 + j / NAPPLY, row block
+// j % NAPPLY; launch 0 applies chunk 0 only); NCONV workgroups writing token
+// images. Launches below 0 only prepare sums and images.
 // Head m runs on XCD m % 8 (its roles share that L2); each XCD issues the
-// roles of its heads role-major in that order, longest first.
+// roles of its heads role-major in that order.
+__host__ __device__ constexpr int n_roles(int parts) { return (2 * parts - 1) * NSTATE + KG * NAPPLY + NCONV; }
+
 template <typename T>
 __global__ __launch_bounds__(PT, 2) void poly_chunk_kernel(PolyArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[kSmemBytes];
   const int x = blockIdx.x % kNumXcd, k = blockIdx.x / kNumXcd;
   const int nh = x < a.M ? (a.M - x + kNumXcd - 1) / kNumXcd : 0;  // heads on this XCD
-  if (k >= nh * NROLE) return;
-  const int rr = k / nh;
+  if (k >= nh * n_roles(a.parts)) return;
+  int rr = k / nh;
   const int m = x + kNumXcd * (k % nh);
   if (a.flags != nullptr && a.flags[m] == 0) return;
   const int b = m / a.H, h = m % a.H;
   char* ws = a.ws + size_t(m) * kPerHead;
-  if (rr >= NUPD + 1 + KG * NAPPLY) {
-    image_role<T>(a, ws, b, h, rr - (NUPD + 1 + KG * NAPPLY));
-  } else if (a.launch < 0) {
+  const int n_state = (2 * a.parts - 1) * NSTATE;
+  if (rr < n_state) {
+    const bool sum = rr >= a.parts * NSTATE;
+    if (sum) rr -= a.parts * NSTATE;
+    Fold f;
+    if (!make_fold(a, rr / NSTATE, sum, f)) return;
+    if (rr % NSTATE < NUPD) quad_update_role(f, ws, rr % NSTATE, smem);
+    else small_update_role(f, ws, smem);
     return;
-  } else if (rr < NUPD) {
-    quad_update_role(a, ws, rr, smem);
-  } else if (rr == NUPD) {
-    small_update_role(a, ws, smem);
-  } else {
-    const int role = rr - (NUPD + 1);
-    const int g = role / NAPPLY;
+  }
+  rr -= n_state;
+  if (rr >= KG * NAPPLY) {
+    image_role<T>(a, ws, b, h, rr - KG * NAPPLY);
+  } else if (a.launch >= 0) {
+    const int g = rr / NAPPLY;
     const int c = a.launch == 0 ? (g == 0 ? 0 : -1) : KG * (a.launch - 1) + 1 + g;
-    if (c >= 0 && c < a.n_chunks) apply_role<T>(a, ws, b, h, m, c, role % NAPPLY, smem);
+    if (c >= 0 && c < a.n_chunks) apply_role<T>(a, ws, b, h, m, c, rr % NAPPLY, smem);
   }
 }
 
-// Clears what must start at zero in every head's workspace: the fp32 masters
-// and shadow slot 0 (state 0, read by launch 0's apply of chunk 0). Every
-// other slot and the token images are written before they are read. The
-// masters and quad slot 0 are one contiguous range, split over kZeroParts
-// workgroups per head; part 0 also clears the small shadows' slot 0.
-constexpr int kZeroParts = 8;
-constexpr size_t kZeroMain = kQuadShadow + size_t(PD) * PD * PD * 2;  // masters + quad slot 0
-
-__device__ __forceinline__ void zero_range(uint8_t* p, size_t bytes, size_t lane, size_t lanes) {
-  float4_t* q = reinterpret_cast<float4_t*>(p);
-  for (size_t i = lane; i < bytes / 16; i += lanes) q[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-}
-
-__global__ void zero_state_kernel(uint8_t* ws, int M) {
-  const int m = blockIdx.x / kZeroParts, part = blockIdx.x % kZeroParts;
-  if (m >= M) return;
-  uint8_t* h = ws + size_t(m) * kPerHead;
-  constexpr size_t kSlice = kZeroMain / kZeroParts;
-  static_assert(kZeroMain % (16 * kZeroParts) == 0, "slices of whole float4s");
-  zero_range(h + part * kSlice, kSlice, threadIdx.x, blockDim.x);
-  if (part == 0) {
-    zero_range(h + kLinShadow, size_t(PD) * PD * 2, threadIdx.x, blockDim.x);
-    zero_range(h + kGramShadow, size_t(PD) * PD * 2, threadIdx.x, blockDim.x);
-    zero_range(h + kZsShadow, 128 * 4, threadIdx.x, blockDim.x);
-  }
-}
+// Parts of a window by the number of heads M. Two parts while the update
+// chain sets the time, one where the chip is busy anyway (polynomial rows
+// alone, us with one / two / four parts, fp32 unless said: 1 head of 100 000 tokens
+// 1687 / 1110 / 1183, 2 of 60 000 1036 / 720 / 728, 8 of 60 000 1113 / 798 /
+// 815, 16 of 30 000 687 / 693 / 719, 24 of 40 000 1079 / 1246 / 1390, 64 of
+// 65536 4388 / 5259 / 5967; four parts are never worth their sums).
+int parts_for(int M) { return M < 16 ? 2 : 1; }
 
 template <typename T>
 int run(PolyArgs a, size_t ws_bytes, hipStream_t stream) {
   (void)ws_bytes;
-  hipLaunchKernelGGL(zero_state_kernel, dim3(unsigned(a.M * kZeroParts)), dim3(256), 0, stream,
-                     reinterpret_cast<uint8_t*>(a.ws), a.M);
-  if (hipGetLastError() != hipSuccess) return TJ_ERR_LAUNCH;
-  const dim3 grid(unsigned(kNumXcd * ((a.M + kNumXcd - 1) / kNumXcd) * NROLE));
-  if (a.n_chunks > 1) {  // token images of the chunks launch 0 folds in
-    a.launch = -1;
+  a.parts = parts_for(a.M);
+  const dim3 grid(unsigned(kNumXcd * ((a.M + kNumXcd - 1) / kNumXcd) * n_roles(a.parts)));
+  // Token images and part sums of the first windows.
+  for (int L = a.n_chunks > 1 ? -image_lag(a.parts) : 0; L < 0; ++L) {
+    a.launch = L;
     hipLaunchKernelGGL(poly_chunk_kernel<T>, grid, dim3(PT), 0, stream, a);
     if (hipGetLastError() != hipSuccess) return TJ_ERR_LAUNCH;
   }
@@ -968,7 +1013,7 @@ extern "C" int tj_poly_attn_fwd(const void* q, const void* k, const void* v, voi
   if (D != tj::PD || chunk != tj::PC) return TJ_ERR_UNSUPPORTED;
   if (B == 0 || S == 0 || exact_prefix >= S) return TJ_OK;
   if (S >= (int64_t(1) << 30) ||
-      !tjh::product_below((int64_t(1) << 31) / tj::NROLE - tj::kNumXcd, {B, H}))
+      !tjh::product_below((int64_t(1) << 31) / tj::n_roles(1) - tj::kNumXcd, {B, H}))
     return TJ_ERR_SHAPE;
   if (!q || !k || !v || !o || !coeffs) return TJ_ERR_SHAPE;
   if (!tjh::view_ok(q, q_strides, dtype) || !tjh::view_ok(k, k_strides, dtype) ||
