@@ -33,8 +33,8 @@
 //     P > 1): the same folding from zero, without shadows, into an fp32 sum.
 //   * token images (KG per head): b = k*sqrt(scale) and v of a later window
 //     (L + 1; L + 2 when P > 1), converted once to fp16 tiles laid out as
-//     the update roles' LDS image, which those roles then stream with direct
-//     global->LDS copies.
+//     the LDS image the state roles and the applies' diagonal blocks then
+//     stream with direct global->LDS copies.
 // State c (before chunk c) lives in shadow slot c % (2 KG): a launch reads
 // the slots of states KG L - KG + 1 .. KG L and writes those of KG L + 1 ..
 // KG L + KG, so applies and updates of one launch never touch the same slot.
@@ -67,7 +67,6 @@ constexpr int NCONV = KG;      // token-image workgroups per head (one chunk eac
 constexpr int NSTATE = NUPD + 1;  // state-update workgroups per head and part
 constexpr int PMAX = 2;        // most parts of a window
 constexpr int NIMG = 4;        // token-image buffers: window w in buffer w % NIMG
-constexpr int LP = 72;         // padded LDS row of 64 halves (144 bytes)
 constexpr int kBufferFlags = 0x00020000;  // raw (untyped) buffer resource word 3 on gfx950
 
 // One state (byte offsets): S_quad without the j < 32 blocks of i >= 32, which
@@ -104,13 +103,12 @@ constexpr uint32_t kTokImgBytes = uint32_t(KG) * (PC / 64) * kTileImg;  // one w
 constexpr uint32_t kTokImg = (kZsShadow + NSLOT * 128 * 4 + 255) & ~255u;  // [NIMG][kTokImgBytes]
 constexpr size_t kPerHead = size_t(kTokImg) + NIMG * kTokImgBytes;
 
-// LDS: apply = quad-state ring (49152) or diagonal tiles (36864);
-//      updates = two transposed token tiles, double buffered (36864).
+// LDS: apply = quad-state ring, then token tiles; updates = token tiles
+// (three stages of 16 KiB each).
 constexpr int kRing = 3;                        // quad-state stages in flight
 constexpr int kRingStage = 2 * PD * PD * 2;     // one stage: rows of two i, [2][64 v][64 j] fp16
 constexpr int kStageBytes = kRing * kRingStage;
 static_assert(kPerHead < (size_t(1) << 31), "workspace offsets of one head fit a buffer resource");
-static_assert(kStageBytes >= 4 * 64 * LP * 2, "diagonal / update tiles must fit the ring area");
 constexpr int kSmemBytes = kStageBytes;
 
 struct PolyArgs {
@@ -222,28 +220,49 @@ struct TokTile {
           half4_t{(half_t)vx[0][e], (half_t)vx[1][e], (half_t)vx[2][e], (half_t)vx[3][e]};
     }
   }
-  // K row-major, V transposed in key_slot order: the diagonal block (as in the exact kernel).
-  __device__ __forceinline__ void store_diag(half_t (*kb)[LP], half_t (*vt)[LP], float rs, int tid) const {
-    int g, c;
-    coords(tid, g, c);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      half4_t hk = {(half_t)((float)kx[r][0] * rs), (half_t)((float)kx[r][1] * rs), (half_t)((float)kx[r][2] * rs),
-                    (half_t)((float)kx[r][3] * rs)};
-      *reinterpret_cast<half4_t*>(&kb[4 * g + r][4 * c]) = hk;
-    }
-    const int slot = key_slot(4 * g);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      half4_t hv = {(half_t)vx[0][e], (half_t)vx[1][e], (half_t)vx[2][e], (half_t)vx[3][e]};
-      *reinterpret_cast<half4_t*>(&vt[4 * c + e][slot]) = hv;
-    }
-  }
 };
 
 // x * s as four packed multiplies. (Element by element the compiler emits
 // eight scalar multiplies and four packs.)
 __device__ __forceinline__ half8_t mul8(half8_t x, half_t s) { return x * half8_t{s, s, s, s, s, s, s, s}; }
+
+// Three LDS stages of one token image each.
+struct TokRing {
+  char s0[kTileImg];
+  char s1[kTileImg];
+  char s2[kTileImg];
+};
+static_assert(sizeof(TokRing) <= kStageBytes, "the token ring must fit the ring area");
+
+// Tokens 8 pc .. 8 pc + 7 of dim row `row` of a tile image.
+__device__ __forceinline__ half8_t img_piece(const half_t* base, int row, int pc) {
+  return *reinterpret_cast<const half8_t*>(reinterpret_cast<const char*>(base) + row * 128 + 16 * (pc ^ ((row >> 1) & 7)));
+}
+
+// Eight dims d0 .. d0 + 7 (d0 = 16 ks + 8 (lane / 32)) of one token of a b^T
+// image per lane: the A operand of a score MFMA, by two transposing reads (16
+// lanes read 4 dim rows of 16 tokens and get one token's 4 dims each). Lane
+// row rho = lane % 32 gets token tok0 + rho with bits 2 and 3 of rho swapped,
+// so that accumulator element r of the scores holds token tok0 + 16 (r / 8) +
+// 8 (lane / 32) + r % 8: eight consecutive tokens per 16-token step, the k-slots
+// that img_piece gives the V^T operand.
+__device__ __forceinline__ half8_t img_tokens(const half_t* bT, int tok0, int ks) {
+  using s4 = short __attribute__((ext_vector_type(4)));
+  using u4 = half4_t;
+  const int lane = threadIdx.x % kWave, i = lane % 16, m = i % 4;
+  const int tok = tok0 + (lane & 16) + 4 * (((m & 1) << 1) | (m >> 1));
+  half8_t r;
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int d = 16 * ks + 8 * (lane / 32) + 4 * x + i / 4;
+    const char* p = reinterpret_cast<const char*>(bT) + d * 128 + 16 * ((tok >> 3) ^ ((d >> 1) & 7)) + 2 * (tok & 4);
+    const u4 v = __builtin_bit_cast(
+        u4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)const_cast<char*>(p)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[4 * x + j] = v[j];
+  }
+  return r;
+}
 
 // ---------------------------------------------------------------------------
 // Apply role: rows [row0, row0 + 256) of the chunk; each wave owns RB = 2
@@ -257,9 +276,6 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
   const int t0 = c * PC, t1 = min(a.S, t0 + PC), slot = c % NSLOT;
   const int row0 = t0 + 4 * WROWS * qt;
   if (row0 >= t1 || row0 + 4 * WROWS <= a.prefix_end) return;
-  auto kb = reinterpret_cast<half_t(*)[64][LP]>(smem);                  // diag: [2][64][LP]
-  auto vt = reinterpret_cast<half_t(*)[64][LP]>(smem + 2 * 64 * LP * 2);  // diag: [2][64][LP]
-
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave, hl = lane / 32, ln = lane % 32;
   const int qw0 = row0 + WROWS * w;
 
@@ -411,6 +427,29 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
     static_for<0, kSteps>(step);
   }
 
+  // Exact diagonal block: keys [t0, min(t1, row0 + 256)), no max subtraction;
+  // the weighted values accumulate straight into accq. The chunk's token
+  // images, written by an earlier launch for the state updates, serve as its
+  // K and V tiles through the same LDS area (fp32 K and V read again and
+  // converted by every apply: 20 of its 69 us, and 2 GB per call of the
+  // extreme workload). The first two copies go out before the linear terms.
+  const int key_end = min(t1, row0 + 4 * WROWS);
+  const int n_kt = (key_end - t0 + 63) / 64;
+  const uint32_t img = kTokImg + uint32_t(c / KG % NIMG) * kTokImgBytes + uint32_t(c % KG) * (PC / 64) * kTileImg;
+  TokRing& tiles = *reinterpret_cast<TokRing*>(smem);
+  auto tile_ptr = [&](auto st) -> char* {
+    if constexpr (decltype(st)::value == 0) return tiles.s0;
+    else if constexpr (decltype(st)::value == 1) return tiles.s1;
+    else return tiles.s2;
+  };
+  auto issue_tile = [&](int kt, auto st) {
+#pragma unroll
+    for (int it = 0; it < 4; ++it)
+      copy_to_lds(rws, tile_ptr(st) + (4 * it + w) * 1024, lane * 16, img + kt * kTileImg + (4 * it + w) * 1024);
+  };
+  issue_tile(0, std::integral_constant<int, 0>{});
+  if (n_kt > 1) issue_tile(1, std::integral_constant<int, 1>{});
+
   // Linear numerator term S_lin^T a^T and the quadratic denominator G a^T
   // (operands straight from the L2-resident shadows). G's rows are read in
   // the order that swaps bits 2 and 3 of the row index, so that accumulator
@@ -454,58 +493,65 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) den_q[rb] = pair_sum(den_q[rb]);
 
-  // Exact diagonal block: keys [t0, min(t1, row0 + 256)), no max subtraction;
-  // the weighted values accumulate straight into accq.
-  const int key_end = min(t1, row0 + 4 * WROWS);
-  const int n_kt = (key_end - t0 + 63) / 64;
-  TokTile<T> tile;
-  tile.init(a, b, h, tid);
-  tile.load(t0);
-  tile.store_diag(kb[0], vt[0], a.rs, tid);
-  __syncthreads();
-  for (int kt = 0; kt < n_kt; ++kt) {
-    const int cur = kt & 1;
-    const int kv0 = t0 + 64 * kt;
-    if (kt + 1 < n_kt) tile.load(kv0 + 64);
+  // Tile kt + 1 (this wave's four copies) must have landed before the barrier.
+  auto wait_tile = [&](int kt) {
+    if (kt + 2 < n_kt) __builtin_amdgcn_s_waitcnt(0x0074);  // vmcnt(4) lgkmcnt(0)
+    else __builtin_amdgcn_s_waitcnt(0x0070);                // vmcnt(0) lgkmcnt(0)
+    lds_barrier();
+  };
+  auto diag_tile = [&](int kt, auto st) {
+    constexpr int sv = decltype(st)::value;
+    if (kt + 2 < n_kt) issue_tile(kt + 2, std::integral_constant<int, (sv + 2) % 3>{});
+    const half_t* bT = reinterpret_cast<const half_t*>(tile_ptr(st));
+    const half_t* vT = bT + PD * 64;
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const int qb0 = qw0 + 32 * rb;
-      const int qi = qb0 + ln;
-      // a block whose rows all precede the tile (or lie past the chunk) skips it
-      if (kv0 <= min(qb0 + 31, key_end - 1)) {
-        float16_t s[2];
+    for (int kh = 0; kh < 2; ++kh) {
+      const int k0 = t0 + 64 * kt + 32 * kh;
+      // Rows that all precede the 32 keys skip them.
+      if (k0 > min(qw0 + WROWS - 1, key_end - 1)) continue;
+      half8_t kf[4], vf[2][2];
 #pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
+      for (int ks = 0; ks < 4; ++ks) kf[ks] = img_tokens(bT, 32 * kh, ks);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) s[kh][r] = 0.f;
+      for (int x = 0; x < 2; ++x)
 #pragma unroll
-          for (int ks = 0; ks < 4; ++ks) {
-            const half8_t kf = *reinterpret_cast<const half8_t*>(&kb[cur][32 * kh + ln][16 * ks + 8 * hl]);
-            s[kh] = mfma32(kf, aB[rb][ks], s[kh]);
-          }
+        for (int vb = 0; vb < 2; ++vb) vf[x][vb] = img_piece(vT, 32 * vb + ln, 4 * kh + 2 * x + hl);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const int qb0 = qw0 + 32 * rb;
+        if (k0 > min(qb0 + 31, key_end - 1)) continue;
+        float16_t sc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) sc = mfma32(kf[ks], aB[rb][ks], sc);
+        half8_t pf[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pf[r / 8][r % 8] = (half_t)fast_exp2(sc[r] * 1.4426950408889634f);
+        if (k0 + 31 > qb0) {  // the causal edge crosses this block
+          const int lim = qb0 + ln - k0 - 8 * hl;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (16 * (r / 8) + r % 8 > lim) pf[r / 8][r % 8] = (half_t)0.f;
         }
-        half8_t pf[4];
+        // den sums the rounded weights, as the value product multiplies them.
 #pragma unroll
-        for (int kh = 0; kh < 2; ++kh)
+        for (int r = 0; r < 16; r += 2)
+          den_d[rb] = __builtin_amdgcn_fdot2(half2_t{pf[r / 8][r % 8], pf[r / 8][r % 8 + 1]},
+                                             half2_t{(half_t)1.f, (half_t)1.f}, den_d[rb], false);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = kv0 + 32 * kh + 8 * (r / 4) + 4 * hl + (r % 4);
-            const float wgt = key <= qi ? fast_exp2(s[kh][r] * 1.4426950408889634f) : 0.f;
-            const half_t wh = (half_t)wgt;
-            den_d[rb] += (float)wh;
-            pf[2 * kh + r / 8][r % 8] = wh;
-          }
+        for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int st = 0; st < 4; ++st)
-#pragma unroll
-          for (int vb = 0; vb < 2; ++vb) {
-            const half8_t vf = *reinterpret_cast<const half8_t*>(&vt[cur][32 * vb + ln][16 * st + 8 * hl]);
-            accq[rb][vb] = mfma32(vf, pf[st], accq[rb][vb]);
-          }
+          for (int vb = 0; vb < 2; ++vb) accq[rb][vb] = mfma32(vf[x][vb], pf[x], accq[rb][vb]);
       }
     }
-    if (kt + 1 < n_kt) tile.store_diag(kb[cur ^ 1], vt[cur ^ 1], a.rs, tid);
-    __syncthreads();
+    wait_tile(kt);
+  };
+  wait_tile(-1);
+  for (int kt = 0; kt < n_kt; kt += 3) {
+    diag_tile(kt, std::integral_constant<int, 0>{});
+    if (kt + 1 < n_kt) diag_tile(kt + 1, std::integral_constant<int, 1>{});
+    if (kt + 2 < n_kt) diag_tile(kt + 2, std::integral_constant<int, 2>{});
   }
 
 #pragma unroll
@@ -553,18 +599,6 @@ __device__ __forceinline__ void apply_role(const PolyArgs& a, const char* ws, in
 // before them) that the barrier needs. The stages are
 // distinct members addressed with compile-time indices, so the compiler can
 // tell the copies into one stage from the reads of another.
-struct TokRing {
-  char s0[kTileImg];
-  char s1[kTileImg];
-  char s2[kTileImg];
-};
-static_assert(sizeof(TokRing) <= kStageBytes, "the token ring must fit the ring area");
-
-// Tokens 8 pc .. 8 pc + 7 of dim row `row` of a tile image.
-__device__ __forceinline__ half8_t img_piece(const half_t* base, int row, int pc) {
-  return *reinterpret_cast<const half8_t*>(reinterpret_cast<const char*>(base) + row * 128 + 16 * (pc ^ ((row >> 1) & 7)));
-}
-
 template <typename Load, typename Mma, typename ChunkEnd>
 __device__ __forceinline__ void stream_image(const char* ws, uint32_t img, int n_chunk, char* smem, Load&& load,
                                              Mma&& mma, ChunkEnd&& chunk_end) {
@@ -901,7 +935,7 @@ template <typename T>
 __device__ void image_role(const PolyArgs& a, char* ws, int b, int h, int j) {
   const int win = a.launch + image_lag(a.parts);
   const int c = KG * win + j;
-  if (c >= a.n_chunks - 1) return;
+  if (c >= a.n_chunks) return;
   char* dst = ws + kTokImg + uint32_t(win % NIMG) * kTokImgBytes + uint32_t(j) * (PC / 64) * kTileImg;
   const int tid = threadIdx.x;
   TokTile<T> x0, x1;
@@ -971,7 +1005,8 @@ int run(PolyArgs a, size_t ws_bytes, hipStream_t stream) {
   a.parts = parts_for(a.M);
   const dim3 grid(unsigned(kNumXcd * ((a.M + kNumXcd - 1) / kNumXcd) * n_roles(a.parts)));
   // Token images and part sums of the first windows.
-  for (int L = a.n_chunks > 1 ? -image_lag(a.parts) : 0; L < 0; ++L) {
+  for (int L = -image_lag(a.parts); L < 0; ++L) {
+    if (L > -image_lag(a.parts) && a.n_chunks == 1) continue;
     a.launch = L;
     hipLaunchKernelGGL(poly_chunk_kernel<T>, grid, dim3(PT), 0, stream, a);
     if (hipGetLastError() != hipSuccess) return TJ_ERR_LAUNCH;
