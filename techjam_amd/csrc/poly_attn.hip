@@ -753,32 +753,55 @@ __device__ __forceinline__ bool make_fold(const PolyArgs& a, int p, bool sum, Fo
   return true;
 }
 
-// NI i-slices per wave, j-blocks JB0..1 (the apply never reads j < 32 for
-// i >= 32: S is symmetric).
-template <int NI, int JB0>
-__device__ __forceinline__ void quad_update_body(const Fold& f, char* ws, int i0, char* smem) {
-  constexpr int NJ = 2 - JB0;
+// One wave folds four slices i0 .. i0 + 3 on one 32-row j-block: eight MFMAs
+// per 16-token step from four LDS reads -- b_j, two of v, and one that gives
+// lane l the piece of slice i0 + l % 4, whose four values are then spread
+// over each row of 16 lanes by DPP moves. The LDS reads, 16 cycles each for
+// the whole CU, are what bounds a tile: with two slices on two j-blocks (or
+// four on one) and each slice's piece read by itself it took 6 (7) reads,
+// 1536 (1792) cycles a workgroup against 1024 of MFMA.
+__device__ __forceinline__ half8_t row_bcast(half8_t x, int i) {
+  using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
+  const u32x4 u = __builtin_bit_cast(u32x4, x);
+  u32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    switch (i) {  // DPP row_newbcast:i
+      case 0: r[e] = __builtin_amdgcn_update_dpp(0, u[e], 0x150, 0xf, 0xf, true); break;
+      case 1: r[e] = __builtin_amdgcn_update_dpp(0, u[e], 0x151, 0xf, 0xf, true); break;
+      case 2: r[e] = __builtin_amdgcn_update_dpp(0, u[e], 0x152, 0xf, 0xf, true); break;
+      default: r[e] = __builtin_amdgcn_update_dpp(0, u[e], 0x153, 0xf, 0xf, true); break;
+    }
+  }
+  return __builtin_bit_cast(half8_t, r);
+}
+
+// Workgroups 0 .. 3: i < 32, one j-block per half; 4 and 5: i >= 32, j >= 32
+// only (the apply never reads j < 32 there: S is symmetric).
+__device__ __forceinline__ void quad_update_role(const Fold& f, char* ws, int ug, char* smem) {
+  constexpr int NI = 4;
   struct Ops {
-    half8_t bj[NJ], vv[2], bi[NI];
+    half8_t bj, vv[2], bi;
   };
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int lane = threadIdx.x % kWave, hl = lane / 32, ln = lane % 32;
-  // acc[ii][jj][vb] = D[j][v] block (jb = JB0 + jj) of S_{i0+ii}. The fp32
-  // state stays in these registers across the fold's chunks.
-  float16_t acc[NI][NJ][2];
+  const int i0 = ug < 4 ? 16 * (ug >> 1) + 4 * w : 32 + 16 * (ug - 4) + 4 * w;
+  const int jb = ug < 4 ? ug & 1 : 1;
+  // acc[ii][vb] = D[j][v] block of S_{i0+ii}. The fp32 state stays in these
+  // registers across the fold's chunks.
+  float16_t acc[NI][2];
   auto blocks = [&](auto&& g) {
 #pragma unroll
     for (int ii = 0; ii < NI; ++ii)
 #pragma unroll
-      for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-        for (int vb = 0; vb < 2; ++vb) g(i0 + ii, JB0 + jj, vb, acc[ii][jj][vb]);
+      for (int vb = 0; vb < 2; ++vb) g(i0 + ii, vb, acc[ii][vb]);
   };
-  blocks([](int, int, int, float16_t& x) {
+  blocks([](int, int, float16_t& x) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) x[r] = 0.f;
   });
   f.sources(ws, [&](const char* st) {
-    blocks([&](int i, int jb, int vb, float16_t& x) { add_img(st + quad_img(i, jb, vb), x); });
+    blocks([&](int i, int vb, float16_t& x) { add_img(st + quad_img(i, jb, vb), x); });
   });
 
   stream_image(
@@ -786,46 +809,43 @@ __device__ __forceinline__ void quad_update_body(const Fold& f, char* ws, int i0
       [&](const half_t* bT, const half_t* vT, int ks) {
         const int pc = 2 * ks + hl;  // tokens 16 ks + 8 hl .. +7 of the tile
         Ops o;
-#pragma unroll
-        for (int jj = 0; jj < NJ; ++jj) o.bj[jj] = img_piece(bT, 32 * (JB0 + jj) + ln, pc);
+        o.bi = img_piece(bT, i0 + (lane & 3), pc);
+        o.bj = img_piece(bT, 32 * jb + ln, pc);
 #pragma unroll
         for (int x = 0; x < 2; ++x) o.vv[x] = img_piece(vT, 32 * x + ln, pc);
-#pragma unroll
-        for (int ii = 0; ii < NI; ++ii) o.bi[ii] = img_piece(bT, i0 + ii, pc);
         return o;
       },
       [&](const Ops& o) {
+        // Issue order: the eight VALU operations of slice ii + 1's product go
+        // four and four after slice ii's two MFMAs. A wave issues in order, so
+        // behind both MFMAs they would wait for the second to leave the pipe
+        // and then hold up the third.
+        half8_t phi = o.bj * row_bcast(o.bi, 0);
 #pragma unroll
-        for (int ii = 0; ii < NI; ++ii)
+        for (int ii = 0; ii < NI; ++ii) {
+          acc[ii][0] = mfma32(phi, o.vv[0], acc[ii][0]);
+          acc[ii][1] = mfma32(phi, o.vv[1], acc[ii][1]);
+          if (ii + 1 < NI) phi = o.bj * row_bcast(o.bi, ii + 1);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);  // VALU
 #pragma unroll
-          for (int jj = 0; jj < NJ; ++jj) {
-            half8_t phi;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) phi[j] = o.bj[jj][j] * o.bi[ii][j];
-#pragma unroll
-            for (int vb = 0; vb < 2; ++vb) acc[ii][jj][vb] = mfma32(phi, o.vv[vb], acc[ii][jj][vb]);
-          }
+        for (int x = 0; x < 2 * (NI - 1); ++x) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
       },
       [&](int j) {
         // fp16 shadow of state_{c+1} for the applies of the next launch: only
         // the pieces the apply reads.
         if (!f.shadow) return;
         char* sh = ws + kQuadShadow + uint32_t((f.c0 + j + 1) % NSLOT) * kShadowBytes;
-        blocks([&](int i, int jb, int vb, const float16_t& x) {
+        blocks([&](int i, int vb, const float16_t& x) {
           store_quad_shadow(reinterpret_cast<half_t*>(sh + quad_shadow(i)), x, jb, vb, 2 * (i >> 4));
         });
       });
   if (f.dst != 0xffffffffu)
-    blocks([&](int i, int jb, int vb, const float16_t& x) { store_img(ws + f.dst + quad_img(i, jb, vb), x); });
-}
-
-// Quad-update workgroups 0..3: i < 32, two slices per wave, both j-blocks;
-// workgroups 4..5: i >= 32, four slices per wave, j >= 32 only -- the same
-// MFMA count per wave.
-__device__ __forceinline__ void quad_update_role(const Fold& f, char* ws, int ug, char* smem) {
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  if (ug < 4) quad_update_body<2, 0>(f, ws, 8 * ug + 2 * w, smem);
-  else quad_update_body<4, 1>(f, ws, 32 + 16 * (ug - 4) + 4 * w, smem);
+    blocks([&](int i, int vb, const float16_t& x) { store_img(ws + f.dst + quad_img(i, jb, vb), x); });
 }
 
 // One wave each: S_lin[j][v] = sum_t b_tj v_tv, G[i][j] = sum_t b_ti b_tj (as
