@@ -317,6 +317,45 @@ int tj_bias_residual_layernorm(float* out, void* ln_out, int ln_dtype, const flo
                                const int32_t* valid_len, int mode, float eps,
                                int zero_ln_padded, hipStream_t stream);
 
+/*
+ * Dense layers on bf16 MFMAs in the split form v = hi + lo (three products
+ * hi.hi + hi.lo + lo.hi, fp32 accumulation): the arithmetic of the GEMM
+ * library's fast float32 mode, for the sizes where that library is slower.
+ * They stand in for the block's projections and the passes that follow them
+ * (torch_transformer_benchmark.py:75-145).
+ *
+ *   out_i[M, N] = x[M, K] w_i[N, K]^T  for the one to three weights given (w1,
+ * w2 and their outputs may be NULL), or, with act 1 (exact GELU) or 2 (ReLU),
+ * one weight and a bias, out = act(x w^T + bias).
+ * narrow 0 runs 32 x 32 output tiles with K split over a workgroup's waves (N
+ * a multiple of 32, K of 64; few rows), narrow 1 the kernel for N = K = 128
+ * (any number of rows, act 0). All tensors fp32, row-major, contiguous,
+ * 16-byte aligned; no output may overlap x.
+ */
+int tj_linear(const float* x, const float* w0, const float* w1, const float* w2,
+              float* out0, float* out1, float* out2, int64_t M, int64_t N, int64_t K,
+              const float* bias, int act, int narrow, hipStream_t stream);
+
+/*
+ * Width 128: the residual forms of tj_bias_residual_layernorm (same modes,
+ * norm and zero_ln_padded; out may be NULL) with y = x w^T, x [M, 128] and w
+ * [128, 128], in one pass. out may be resid itself; otherwise no output may
+ * overlap an input or another output.
+ */
+int tj_narrow_residual_norm(const float* x, const float* w, const float* bias, const float* resid, float* out,
+                            int64_t M, int64_t seq_len, const int32_t* valid_len, int mode,
+                            const float* gamma, const float* beta, float* ln_out, float eps,
+                            int zero_ln_padded, hipStream_t stream);
+
+/*
+ * The same with y = act(x w_in^T + bias_in) w_out^T (act 1 exact GELU, 2
+ * ReLU), both weights [128, 128]: the FFN half of a block of width 128.
+ */
+int tj_narrow_ffn_norm(const float* x, const float* w_in, const float* bias_in, int act, const float* w_out,
+                       const float* bias, const float* resid, float* out, int64_t M, int64_t seq_len,
+                       const int32_t* valid_len, int mode, const float* gamma, const float* beta,
+                       float* ln_out, float eps, int zero_ln_padded, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -75,6 +75,11 @@ SIGNATURES = {
         _int,
         [_vp, _vp, _int, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _int, _f32, _int, _vp],
     ),
+    "tj_linear": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _int, _int, _vp]),
+    "tj_narrow_residual_norm": (
+        _int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _int, _vp, _vp, _vp, _f32, _int, _vp]),
+    "tj_narrow_ffn_norm": (
+        _int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _int, _vp, _vp, _vp, _f32, _int, _vp]),
     "tj_quad_apply": (
         _int,
         [_vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p, _vp],

@@ -20,6 +20,7 @@ import torch.nn.functional as F
 
 from .kernels.attention import scaled_dot_product_attention
 from .kernels.elementwise import NORM_WIDTHS
+from .kernels.linear import ffn_norm, projections, residual_norm
 
 
 ACTIVATIONS = ("gelu", "relu")
@@ -118,7 +119,8 @@ def project(x: torch.Tensor, weight: torch.Tensor, owner: nn.Module, key: str,
     float16 ``x`` runs on fp16 operands (the weight's cached fp16 copy) with
     fp32 accumulation, its result in ``out_dtype`` (default float16)."""
     if x.dtype != torch.float16:
-        return _linear_f32(x, weight)
+        own = projections(x, (weight,))
+        return _linear_f32(x, weight) if own is None else own[0]
     w16 = fp16_weight(owner, key, weight)
     if out_dtype in (None, torch.float16):
         return F.linear(x, w16)
@@ -172,6 +174,9 @@ class HipSelfAttention(nn.Module):
     def project_qkv_folded(self, x: torch.Tensor):
         """Bias-free q, k, v head views (fp16 for an fp16 ``x``) and the q / v
         biases the kernel adds (a key bias never changes the attention output)."""
+        own = projections(x, (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight))
+        if own is not None:  # one launch
+            return (*map(self.heads_view, own), self.q_proj.bias, self.v_proj.bias)
         return (self.heads_view(project(x, self.q_proj.weight, self.q_proj, "weight")),
                 self.heads_view(project(x, self.k_proj.weight, self.k_proj, "weight")),
                 self.heads_view(project(x, self.v_proj.weight, self.v_proj, "weight")),
@@ -252,6 +257,13 @@ class EncoderBlock(nn.Module):
                 and all(type(n) is nn.LayerNorm and n.elementwise_affine and n.bias is not None
                         and n.weight.dtype == torch.float32 for n in (self.norm1, self.norm2)))
 
+    def _hidden(self, a, act):
+        """The FFN's fp32 hidden activations, ``act(ffn_in(a))``."""
+        own = projections(a, (self.ffn_in.weight,), self.ffn_in.bias, self.activation)
+        if own is not None:
+            return own[0]
+        return _must(act(_linear_f32(a, self.ffn_in.weight), self.ffn_in.bias))
+
     def _forward_fused(self, x, valid_token_mask, causal, valid_len):
         """Same computation as the unfused forward; the projection GEMMs run
         bias-free and each bias add, residual add, activation and row zeroing
@@ -264,11 +276,10 @@ class EncoderBlock(nn.Module):
         act = bias_gelu if self.activation == "gelu" else bias_relu
         attn = self.attention
         ctx = attn.context(self.norm1(x), valid_token_mask, causal, valid_len)
-        y = _linear_f32(ctx, attn.out_proj.weight)
+        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight")
         x = _must(bias_residual(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, out=y))
-        h = _linear_f32(self.norm2(x), self.ffn_in.weight)
-        _must(act(h, self.ffn_in.bias))
-        y = _linear_f32(h, self.ffn_out.weight)
+        h = self._hidden(self.norm2(x), act)
+        y = project(h, self.ffn_out.weight, self.ffn_out, "weight")
         return _must(bias_residual(x, y, self.ffn_out.bias, valid_len, MODE_ZERO_OUT, out=y))
 
     def _forward_fused_post(self, x, valid_token_mask, causal, valid_len):
@@ -280,14 +291,13 @@ class EncoderBlock(nn.Module):
         act = bias_gelu if self.activation == "gelu" else bias_relu
         attn = self.attention
         ctx = attn.context(x, valid_token_mask, causal, valid_len)
-        y = _linear_f32(ctx, attn.out_proj.weight)
+        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight")
         del ctx
         _, x = _must(bias_residual_layernorm(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, self.norm1,
                                              keep_sum=False))
         del y
-        h = _linear_f32(x, self.ffn_in.weight)
-        _must(act(h, self.ffn_in.bias))
-        y = _linear_f32(h, self.ffn_out.weight)
+        h = self._hidden(x, act)
+        y = project(h, self.ffn_out.weight, self.ffn_out, "weight")
         del h
         _, x = _must(bias_residual_layernorm(x, y, self.ffn_out.bias, valid_len, MODE_PLAIN, self.norm2,
                                              zero_padded_norm=valid_token_mask is not None, keep_sum=False))
@@ -327,16 +337,31 @@ class EncoderBlock(nn.Module):
             a = a.half()
         ctx = attn.context(a, valid_token_mask, causal, valid_len)
         del a
-        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", f32)
-        del ctx
-        x, a = _must(bias_residual_layernorm(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, self.norm2, out=y,
-                                             norm_dtype=f16 if fp16_operands else f32))
-        del y
-        h = project(a, self.ffn_in.weight, self.ffn_in, "weight", f32)
-        del a
-        # the activation in place, or straight into the fp16 operand of the next GEMM
+        # Layers of width 128: a projection and the passes after it in one.
+        own = None if fp16_operands else residual_norm(ctx, attn.out_proj.weight, attn.out_proj.bias, x, valid_len,
+                                                       MODE_ZERO_Y, self.norm2)
+        if own is not None:
+            del ctx
+            x, a = own
+        else:
+            y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", f32)
+            del ctx
+            x, a = _must(bias_residual_layernorm(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, self.norm2, out=y,
+                                                 norm_dtype=f16 if fp16_operands else f32))
+            del y
+        own = None if fp16_operands else ffn_norm(a, self.ffn_in.weight, self.ffn_in.bias, self.activation,
+                                                  self.ffn_out.weight, self.ffn_out.bias, x, valid_len, MODE_ZERO_OUT,
+                                                  next_norm, zero_padded_norm=last and valid_token_mask is not None)
+        if own is not None:
+            return own
         act = bias_gelu if self.activation == "gelu" else bias_relu
-        h = _must(act(h, self.ffn_in.bias, out_f16=fp16_operands))
+        if fp16_operands:
+            h = project(a, self.ffn_in.weight, self.ffn_in, "weight", f32)
+            # the activation straight into the fp16 operand of the next GEMM
+            h = _must(act(h, self.ffn_in.bias, out_f16=True))
+        else:
+            h = self._hidden(a, act)
+        del a
         y = project(h, self.ffn_out.weight, self.ffn_out, "weight", f32)
         del h
         return _must(bias_residual_layernorm(x, y, self.ffn_out.bias, valid_len, MODE_ZERO_OUT, next_norm, out=y,
