@@ -24,7 +24,19 @@ int launch(const AttnArgs& a, hipStream_t stream) {
       if constexpr (HD == 64 && sizeof(T) == 4) return launch_split_wide(a, stream);
     }
   }
-  return launch_qb<T, HD, 1>(a, stream);
+  // Wide fp32 heads on 32-key tiles where 64-key tiles do not fit the
+  // registers: head_dim 256 spilled 49 of its 512 (B=64 H=4 S=128 41.5 -> 32.1
+  // us, B=4 H=16 S=4096 causal 2243 -> 1298 us, not causal 4589 -> 2541), and
+  // split scores at 128 took 363, one wave per SIMD (same shapes 22.8 -> 20.1,
+  // 887 -> 706, 1658 -> 1262). Plain head_dim 128 fits and stays on 64 keys
+  // (413 us against 439 on 32).
+  if constexpr (sizeof(T) == 4 && HD == 256) {
+    return launch_qb<T, HD, 1, 32>(a, stream);
+  } else {
+    if constexpr (sizeof(T) == 4 && HD == 128)
+      if (a.qk_split != nullptr) return launch_qb<T, HD, 1, 32>(a, stream);
+    return launch_qb<T, HD, 1>(a, stream);
+  }
 }
 
 template <typename T>

@@ -9,8 +9,9 @@
 //   * One workgroup = 4 waves = a tile of 128 QB query rows of one (b, h);
 //     each wave owns QB blocks of 32 consecutive rows (QB = 1 or 2) for the
 //     whole key loop.
-//   * Keys stream through LDS in tiles of 64 (32 for the split-score kernel
-//     with two query blocks per wave) -- double buffered: K row-major, V
+//   * Keys stream through LDS in tiles of 64 (32 for the instances whose
+//     registers 64 would exceed: split scores with two query blocks per wave or
+//     at head_dim 128, head_dim 256, fp32 inputs) -- double buffered: K row-major, V
 //     transposed, both converted to fp16 while being stored.
 //   * Scores are computed transposed, S^T = K Q^T (keys x queries), so a lane
 //     holds 32 keys of ONE query: the row max/sum is lane-local plus one swap
@@ -623,7 +624,7 @@ int launch_qb(AttnArgs a, hipStream_t stream) {
   const int64_t per_xcd = (bhn + kNumXcd - 1) / kNumXcd;
   const int64_t grid = a.balanced ? bhn * a.n_mtiles : kNumXcd * (per_xcd + a.group - 1) * a.n_mtiles;
   if (grid * NT >= (int64_t(1) << 32)) return TJ_ERR_SHAPE;
-  if constexpr ((QB == 1 && HD <= 128) || BNT == 32) {
+  if constexpr (HD <= 128 && (QB == 1 || BNT == 32)) {
     if (a.qk_split != nullptr) {
       hipLaunchKernelGGL((attn_fwd_kernel<T, HD, QB, true, BNT>), dim3(uint32_t(grid)), dim3(NT), 0, stream, a);
       return tjh::launch_status();
