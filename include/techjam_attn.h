@@ -116,6 +116,25 @@ int tj_attn_fwd_proj_bias(const void* q, const void* k, const void* v, void* o, 
                           const float* q_bias, const float* v_bias, hipStream_t stream);
 
 /*
+ * tj_attn_fwd / tj_attn_fwd_proj_bias without row limits, with a workspace
+ * (qk_split and either bias may be NULL). With
+ * few query tiles and long key sweeps the launch is otherwise as long as its
+ * longest tile: each tile's keys are then cut into parts, computed side by
+ * side into the workspace and added by a second kernel. tj_attn_workspace_bytes
+ * gives the bytes that takes (16-byte aligned, contents irrelevant, calls
+ * sharing one ordered on one stream), 0 where the parts would not pay;
+ * workspace may then be NULL, and with NULL every sweep runs whole.
+ */
+size_t tj_attn_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D, int causal);
+int tj_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, int dtype,
+                   int64_t B, int64_t H, int64_t S, int64_t D,
+                   const int64_t q_strides[4], const int64_t k_strides[4],
+                   const int64_t v_strides[4], const int64_t o_strides[4],
+                   float scale, int causal, const int32_t* valid_len, const int32_t* qk_split,
+                   const float* q_bias, const float* v_bias,
+                   void* workspace, size_t workspace_bytes, hipStream_t stream);
+
+/*
  * Device-side score guard of the polynomial route.
  *
  * Replaces estimate_sigma / poly_is_safe / hermite_coefficients

@@ -7,6 +7,11 @@
 namespace tj {
 namespace {
 
+// Shortest part, in key tiles, and the tiles a sweep must be longer than a part
+// for the split to pay for the partial sums and the second kernel.
+constexpr int64_t kMinPart = 8;
+constexpr int64_t kPartGain = 12;
+
 // Two query blocks per wave halve LDS operand traffic and staging per MFMA.
 // They fit the register budget for head_dim <= 64 (with split scores only at
 // head_dim 64 with 32-key tiles, fp32 inputs), and need sequences long enough
@@ -39,6 +44,44 @@ int launch(const AttnArgs& a, hipStream_t stream) {
   }
 }
 
+// Key parts, where the longest key sweep of a 128-row query tile is at least
+// 2.5 times what an even split of all key tiles over the chip's workgroup
+// slots gives; part_tiles 0: none. Measured (us, one sweep -> parts, causal,
+// head_dim 64 fp32): 1 head of 2048 33 -> 19, of 8192 114 -> 30, of 16 384 224
+// -> 74; 4 heads of 4096 61 -> 31, 8 of 2048 34 -> 26. Past the line the parts
+// cost as much as they save: 16 heads of 4096 75 -> 73 (head_dim 128 129 ->
+// 135), 32 of 2048 43 -> 47.
+struct PartPlan {
+  int part_tiles = 0, n_parts = 0, n_mtiles = 0;
+};
+
+PartPlan plan_parts(int64_t B, int64_t H, int64_t S, int64_t D, int causal) {
+  PartPlan p;
+  const int64_t nm = (S + 127) / 128, nk = (S + 63) / 64, bhn = B * H;
+  if (bhn * nm > 4096) return p;
+  // Two workgroups on each of 256 CUs; one at head_dim 256.
+  const int64_t slots = D == 256 ? 256 : 512;
+  const int64_t all = bhn * (causal ? nm * (nm + 1) : nm * nk);
+  int64_t part = (all + slots - 1) / slots;
+  part = part < kMinPart ? kMinPart : part;
+  part += part & 1;  // whole 128-row steps
+  if (nk < part + kPartGain || 2 * nk < 5 * part) return p;
+  p.part_tiles = (int)part;
+  p.n_mtiles = (int)nm;
+  p.n_parts = first_part((int)nm, (int)nk, (int)part, causal);
+  return p;
+}
+
+template <typename T>
+int dispatch_parts(const AttnArgs& a, int64_t D, hipStream_t stream) {
+  switch (D) {
+    case 32: return launch_parts<T, 32>(a, stream);
+    case 64: return launch_parts<T, 64>(a, stream);
+    case 128: return launch_parts<T, 128>(a, stream);
+    default: return launch_parts<T, 256>(a, stream);
+  }
+}
+
 template <typename T>
 int dispatch_hd(const AttnArgs& a, int64_t D, hipStream_t stream) {
   switch (D) {
@@ -59,7 +102,7 @@ int attn_fwd(const void* q, const void* k, const void* v, void* o, int dtype, in
              int64_t D, const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
              const int64_t o_strides[4], float scale, int causal, const int32_t* valid_len,
              const int32_t* row_limit, const int32_t* qk_split, const float* q_bias, const float* v_bias,
-             hipStream_t stream) {
+             void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (dtype != TJ_F32 && dtype != TJ_F16) return TJ_ERR_DTYPE;
   if (B < 0 || H <= 0 || S < 0 || D <= 0) return TJ_ERR_SHAPE;
   // Tile indices fit 31 bits; the launch also checks that its grid fits the
@@ -90,6 +133,16 @@ int attn_fwd(const void* q, const void* k, const void* v, void* o, int dtype, in
   a.qk_split = qk_split;
   a.q_bias = q_bias;
   a.v_bias = v_bias;
+  const tj::PartPlan plan = workspace != nullptr ? tj::plan_parts(B, H, S, D, a.causal) : tj::PartPlan();
+  if (plan.part_tiles > 0) {
+    if (workspace_bytes < tj_attn_workspace_bytes(B, H, S, D, causal) || !tjh::aligned16(workspace)) return TJ_ERR_WORKSPACE;
+    a.part_tiles = plan.part_tiles;
+    a.n_parts = plan.n_parts;
+    a.n_mtiles = plan.n_mtiles;
+    a.part_o = static_cast<float*>(workspace);
+    a.part_ml = a.part_o + B * H * plan.n_parts * 128 * D;
+    return dtype == TJ_F32 ? tj::dispatch_parts<float>(a, D, stream) : tj::dispatch_parts<half_t>(a, D, stream);
+  }
   if (dtype == TJ_F32) return tj::dispatch_hd<float>(a, D, stream);
   return tj::dispatch_hd<half_t>(a, D, stream);
 }
@@ -103,7 +156,7 @@ extern "C" int tj_attn_fwd(const void* q, const void* k, const void* v, void* o,
                            float scale, int causal, const int32_t* valid_len,
                            const int32_t* row_limit, const int32_t* qk_split, hipStream_t stream) {
   return attn_fwd(q, k, v, o, dtype, B, H, S, D, q_strides, k_strides, v_strides, o_strides, scale, causal,
-                  valid_len, row_limit, qk_split, nullptr, nullptr, stream);
+                  valid_len, row_limit, qk_split, nullptr, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int tj_attn_fwd_proj_bias(const void* q, const void* k, const void* v, void* o, int dtype,
@@ -113,5 +166,24 @@ extern "C" int tj_attn_fwd_proj_bias(const void* q, const void* k, const void* v
                                      float scale, int causal, const int32_t* valid_len,
                                      const float* q_bias, const float* v_bias, hipStream_t stream) {
   return attn_fwd(q, k, v, o, dtype, B, H, S, D, q_strides, k_strides, v_strides, o_strides, scale, causal,
-                  valid_len, nullptr, nullptr, q_bias, v_bias, stream);
+                  valid_len, nullptr, nullptr, q_bias, v_bias, nullptr, 0, stream);
+}
+
+extern "C" size_t tj_attn_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D, int causal) {
+  if (B <= 0 || H <= 0 || S <= 0 || S >= (int64_t(1) << 30) || (D != 32 && D != 64 && D != 128 && D != 256)) return 0;
+  if (!tjh::product_below(int64_t(1) << 31, {B, H, (S + 127) / 128})) return 0;
+  const tj::PartPlan p = tj::plan_parts(B, H, S, D, causal);
+  if (p.part_tiles == 0) return 0;
+  return size_t(B) * size_t(H) * size_t(p.n_parts) * 128 * size_t(D + 2) * sizeof(float);
+}
+
+extern "C" int tj_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, int dtype,
+                              int64_t B, int64_t H, int64_t S, int64_t D,
+                              const int64_t q_strides[4], const int64_t k_strides[4],
+                              const int64_t v_strides[4], const int64_t o_strides[4],
+                              float scale, int causal, const int32_t* valid_len, const int32_t* qk_split,
+                              const float* q_bias, const float* v_bias,
+                              void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  return attn_fwd(q, k, v, o, dtype, B, H, S, D, q_strides, k_strides, v_strides, o_strides, scale, causal,
+                  valid_len, nullptr, qk_split, q_bias, v_bias, workspace, workspace_bytes, stream);
 }

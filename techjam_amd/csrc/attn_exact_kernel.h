@@ -75,6 +75,11 @@ struct AttnArgs {
   int n_mtiles;
   int group;     // (b, h) per interleaved group on one XCD
   int balanced;  // spread every (b, h) over all XCDs (row limits or B*H < 8)
+  // Key parts (attn_parts_kernel): at most part_tiles key tiles each, n_parts
+  // of them per (b, h); unnormalised outputs and (reference, sum) pairs.
+  int part_tiles, n_parts;
+  float* part_o;   // [B*H*n_parts][128][D]
+  float* part_ml;  // [B*H*n_parts][128][2]
 };
 
 // The split-score kernel with two query blocks per wave on 32-key tiles
@@ -249,9 +254,11 @@ struct KVStage {
 // One query tile of one (b, h): 4 waves x 32*QB rows. Each wave holds QB
 // 32-row query blocks, so every K / V^T operand read from LDS feeds QB MFMAs.
 // SPLIT selects the three-MFMA score path.
-template <typename T, int HD, int QB, bool SPLIT, int BNT, typename SM>
+// PART runs key tiles [kt0, kt0 + a.part_tiles) only; with slot >= 0 the tile
+// has more parts and the result goes to that slot of the part buffers.
+template <typename T, int HD, int QB, bool SPLIT, int BNT, bool PART = false, typename SM>
 __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int h, int q0, int row_cap,
-                                          int L) {
+                                          int L, int kt0 = 0, int64_t slot = -1) {
   using TL = Tile<T, HD>;
   constexpr int NKB = BNT / 32;  // 32-key score blocks per tile
   constexpr int NS = BNT / 16;   // 16-key PV steps per tile
@@ -268,7 +275,8 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
   // by the epilogue); a tile with none of them streams no keys at all.
   const int row_end = min(min(q0 + TROWS, L), row_cap);
   const int kv_end = q0 >= row_end ? 0 : (a.causal ? row_end : L);
-  const int n_kv = kv_end > 0 ? (kv_end + BNT - 1) / BNT : 0;
+  const int n_kv_all = kv_end > 0 ? (kv_end + BNT - 1) / BNT : 0;
+  const int n_kv = PART ? min(n_kv_all, kt0 + a.part_tiles) : n_kv_all;
   // Last key this wave needs (inclusive); waves whose rows are all padding
   // (or beyond row_cap) compute nothing.
   int wave_last_key = a.causal ? min(qw0 + WROWS - 1, kv_end - 1) : kv_end - 1;
@@ -277,7 +285,7 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
   // The first key tile's loads go out before q's, so the two latencies overlap.
   KVStage<T, HD, BNT / 16> stage;
   stage.init(a, b, h, tid);
-  if (n_kv > 0) stage.load(0, tid);
+  if (n_kv > kt0) stage.load(kt0 * BNT, tid);
 
   // Q^T as the B operand: lane holds query qw0 + 32*qb + ln, dims 16*ks + 8*hl .. +7.
   half8_t qf[QB][TL::KS];
@@ -342,18 +350,18 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
       for (int r = 0; r < 16; ++r) oacc[qb][db][r] = 0.f;
   }
 
-  if (n_kv > 0) stage.template store<SPLIT>(sm, 0, tid);
+  if (n_kv > kt0) stage.template store<SPLIT>(sm, 0, tid);
   __syncthreads();
 
-  for (int kt = 0; kt < n_kv; ++kt) {
-    const int cur = kt & 1;
+  for (int kt = kt0; kt < n_kv; ++kt) {
+    const int cur = (kt - kt0) & 1;
     const int kv0 = kt * BNT;
     if (kt + 1 < n_kv) stage.load(kv0 + BNT, tid);
 
     if (kv0 <= wave_last_key) {
       // Scores come out of the MFMA already shifted by the running max: the
       // accumulator starts at -m_run (0 on the first tile, where m_run is set).
-      const bool first = kv0 == 0;
+      const bool first = kt == kt0;
       float16_t sacc[QB][NKB];
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
@@ -490,6 +498,24 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
   for (int qb = 0; qb < QB; ++qb) {
     const int qi = qw0 + 32 * qb + ln;
     const float l_tot = pair_sum(l_run[qb]);
+    if constexpr (PART) {
+      if (slot >= 0) {
+        const int row = qi - q0;
+        float* po = a.part_o + (slot * 128 + row) * HD;
+#pragma unroll
+        for (int db = 0; db < TL::DB; ++db)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<float4_t*>(po + db * 32 + 8 * g + 4 * hl) =
+                float4_t{oacc[qb][db][4 * g], oacc[qb][db][4 * g + 1], oacc[qb][db][4 * g + 2], oacc[qb][db][4 * g + 3]};
+        if (hl == 0) {
+          // A wave without keys in this part leaves sum 0; its reference is not read.
+          a.part_ml[(slot * 128 + row) * 2] = l_tot > 0.f ? m_run[qb] : 0.f;
+          a.part_ml[(slot * 128 + row) * 2 + 1] = l_tot;
+        }
+        continue;
+      }
+    }
     if (qi < row_cap) {
       const bool valid = qi < L && l_tot > 0.f;
       const float inv = valid ? 1.f / l_tot : 0.f;
@@ -612,6 +638,127 @@ __global__ __launch_bounds__(NT, (HD > 128 ? 1 : 2)) void attn_fwd_kernel(AttnAr
     }
   }
   attn_tile<T, HD, QB, false, BNT>(a, sm, b, h, q0, row_cap, L);
+}
+
+// Parts of query tile mt, and the tile and part that position j of a (b, h)'s
+// list is. Causal tile mt (128 rows) has 2 (mt + 1) key tiles of 64, so with
+// c = part_tiles / 2 tiles c g .. c g + c - 1 have g + 1 parts.
+__host__ __device__ inline int tile_parts(int mt, int n_keytiles, int part_tiles, int causal) {
+  return causal ? mt / (part_tiles / 2) + 1 : (n_keytiles + part_tiles - 1) / part_tiles;
+}
+__host__ __device__ inline int first_part(int mt, int n_keytiles, int part_tiles, int causal) {
+  if (!causal) return mt * ((n_keytiles + part_tiles - 1) / part_tiles);
+  const int c = part_tiles / 2, g = mt / c;
+  return c * g * (g + 1) / 2 + (mt - c * g) * (g + 1);
+}
+
+// Few query tiles: each tile's keys are cut into parts of a.part_tiles key
+// tiles, one workgroup each, so that the launch is as long as a part instead
+// of the longest tile (and covers the chip). Tiles of more than one part leave
+// unnormalised sums, which combine_parts_kernel adds. A part starts at a
+// multiple of 128 keys at or before its tile's first row, so every row sees
+// its first key and the running reference is finite.
+template <typename T, int HD, bool SPLIT_OK>
+__global__ __launch_bounds__(NT, (HD > 128 ? 1 : 2)) void attn_parts_kernel(AttnArgs a) {
+  constexpr int BNT = sizeof(T) == 4 && (HD == 256 || (HD == 128 && SPLIT_OK)) ? 32 : 64;
+  __shared__ Smem<HD, SPLIT_OK, BNT> sm;
+  // Each XCD takes a contiguous range of the (b, h)'s lists, so that few XCDs
+  // read one (b, h)'s keys; the last (longest) tiles come first in a list.
+  const int64_t total = int64_t(a.B) * a.H * a.n_parts, per = (total + kNumXcd - 1) / kNumXcd;
+  const int64_t id = (blockIdx.x % kNumXcd) * per + blockIdx.x / kNumXcd;
+  if (blockIdx.x / kNumXcd >= per || id >= total) return;
+  const int bh = (int)(id / a.n_parts), j = a.n_parts - 1 - (int)(id % a.n_parts);
+  const int nk = (a.S + 63) / 64;
+  int mt = 0;
+  if (a.causal) {
+    const int c = a.part_tiles / 2;
+    int g = 0;
+    while (c * (g + 1) * (g + 2) / 2 <= j) ++g;  // group of tiles with g + 1 parts
+    mt = c * g + (j - c * g * (g + 1) / 2) / (g + 1);
+  } else {
+    mt = j / tile_parts(0, nk, a.part_tiles, 0);
+  }
+  const int p = j - first_part(mt, nk, a.part_tiles, a.causal);
+  const bool whole = tile_parts(mt, nk, a.part_tiles, a.causal) == 1;
+  const int b = bh / a.H, h = bh % a.H;
+  int L = a.S;
+  if (a.valid_len != nullptr) L = min(a.S, max(0, a.valid_len[b]));
+  AttnArgs t = a;
+  t.part_tiles = a.part_tiles * (64 / BNT);
+  const int64_t slot = whole ? -1 : int64_t(bh) * a.n_parts + j;
+  if constexpr (SPLIT_OK) {
+    if (a.qk_split[bh] != 0) {
+      attn_tile<T, HD, 1, true, BNT, true>(t, sm, b, h, mt * 128, a.S, L, p * t.part_tiles, slot);
+      return;
+    }
+  }
+  attn_tile<T, HD, 1, false, BNT, true>(t, sm, b, h, mt * 128, a.S, L, p * t.part_tiles, slot);
+}
+
+// Adds the parts of one query tile: out = sum_p 2^(m_p - M) O_p / sum_p
+// 2^(m_p - M) l_p (+ v bias), zero for rows at or past the valid length. One
+// row per HD / 4 lanes and thread, the loads of several parts in flight: with
+// a tile's rows and parts one after another its latency was most of the call.
+template <typename T, int HD>
+__global__ __launch_bounds__(NT) void combine_parts_kernel(AttnArgs a) {
+  constexpr int LPR = HD / 4, RPB = NT / LPR;  // lanes per row, rows per workgroup
+  const int tile = blockIdx.x / (128 / RPB);
+  const int bh = tile / a.n_mtiles, mt = tile % a.n_mtiles;
+  const int nk = (a.S + 63) / 64;
+  const int np = tile_parts(mt, nk, a.part_tiles, a.causal);
+  const int r = blockIdx.x % (128 / RPB) * RPB + threadIdx.x / LPR, qi = mt * 128 + r;
+  if (np == 1 || qi >= a.S) return;
+  const int b = bh / a.H, h = bh % a.H;
+  int L = a.S;
+  if (a.valid_len != nullptr) L = min(a.S, max(0, a.valid_len[b]));
+  const int c = 4 * (threadIdx.x % LPR);
+  float4_t y = {0.f, 0.f, 0.f, 0.f};
+  if (qi < L) {
+    using float2_t = float __attribute__((ext_vector_type(2)));
+    const int64_t slot0 = int64_t(bh) * a.n_parts + first_part(mt, nk, a.part_tiles, a.causal);
+    const float2_t* ml = reinterpret_cast<const float2_t*>(a.part_ml) + slot0 * 128 + r;
+    const float* po = a.part_o + (slot0 * 128 + r) * HD + c;
+    float m = -__builtin_inff();
+#pragma unroll 8
+    for (int p = 0; p < np; ++p) {
+      const float2_t x = ml[p * 128];
+      m = x[1] > 0.f ? fmaxf(m, x[0]) : m;
+    }
+    float l = 0.f;
+#pragma unroll 4
+    for (int p = 0; p < np; ++p) {
+      const float2_t x = ml[p * 128];
+      const float4_t o = *reinterpret_cast<const float4_t*>(po + (int64_t)p * 128 * HD);
+      const float wgt = x[1] > 0.f ? fast_exp2(x[0] - m) : 0.f;  // a part without keys holds zeros
+      l += wgt * x[1];
+      y += wgt * o;
+    }
+    const float4_t bv = a.v_bias != nullptr ? *reinterpret_cast<const float4_t*>(a.v_bias + h * HD + c) : float4_t{0.f, 0.f, 0.f, 0.f};
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = l > 0.f ? y[e] * inv + bv[e] : 0.f;
+  }
+  T* op = reinterpret_cast<T*>(a.o) + a.vo.row(b, h, qi) + c;
+  if constexpr (sizeof(T) == 4) *reinterpret_cast<float4_t*>(op) = y;
+  else *reinterpret_cast<half4_t*>(op) = half4_t{(half_t)y[0], (half_t)y[1], (half_t)y[2], (half_t)y[3]};
+}
+
+template <typename T, int HD>
+int launch_parts(AttnArgs a, hipStream_t stream) {
+  const int64_t bhn = int64_t(a.B) * a.H, total = bhn * a.n_parts;
+  const int64_t grid = (total + kNumXcd - 1) / kNumXcd * kNumXcd;
+  if (a.qk_split == nullptr) {
+    hipLaunchKernelGGL((attn_parts_kernel<T, HD, false>), dim3(uint32_t(grid)), dim3(NT), 0, stream, a);
+  } else if constexpr (HD <= 128) {
+    hipLaunchKernelGGL((attn_parts_kernel<T, HD, true>), dim3(uint32_t(grid)), dim3(NT), 0, stream, a);
+  } else {
+    return TJ_ERR_UNSUPPORTED;
+  }
+  const int rc = tjh::launch_status();
+  if (rc != TJ_OK) return rc;
+  hipLaunchKernelGGL((combine_parts_kernel<T, HD>), dim3(uint32_t(bhn * a.n_mtiles * (HD / 8))), dim3(NT), 0,
+                     stream, a);
+  return tjh::launch_status();
 }
 
 template <typename T, int HD, int QB, int BNT = BN>

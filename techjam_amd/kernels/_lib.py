@@ -51,6 +51,12 @@ SIGNATURES = {
         [_vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p, _i64p,
          _f32, _int, _vp, _vp, _vp, _vp],
     ),
+    "tj_attn_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _i64, _int]),
+    "tj_attn_fwd_ws": (
+        _int,
+        [_vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _i64p, _i64p, _i64p, _i64p,
+         _f32, _int, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp],
+    ),
     "tj_score_guard": (
         _int,
         [_vp, _vp, _int, _i64, _i64, _i64, _i64, _i64p, _i64p, _f32, _vp, _i64, _f32, _i64,

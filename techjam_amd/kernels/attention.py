@@ -183,14 +183,19 @@ def scaled_dot_product_attention(
                                   or not t.is_contiguous() or t.data_ptr() % 16):
                 raise ValueError(f"{name} must be a contiguous, 16-byte aligned float32 tensor of {h * d} "
                                  f"elements on {dev}")
-        code = _lib.lib().tj_attn_fwd_proj_bias(
+    if row_limit is None:
+        # Long sweeps over few query tiles are cut into parts, whose sums need
+        # a workspace; 0 bytes for all other calls.
+        ws_bytes = _lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(bool(is_causal)))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+        code = _lib.lib().tj_attn_fwd_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],
             b, h, s, d,
             _lib.strides4(q), _lib.strides4(k), _lib.strides4(v), _lib.strides4(out),
-            float(scale), int(bool(is_causal)), _ptr(valid_len), _ptr(q_bias), _ptr(v_bias),
-            _stream_ptr(dev),
+            float(scale), int(bool(is_causal)), _ptr(valid_len), _ptr(qk_split), _ptr(q_bias), _ptr(v_bias),
+            _ptr(ws), ws_bytes, _stream_ptr(dev),
         )
-        _lib.check(code, "tj_attn_fwd_proj_bias")
+        _lib.check(code, "tj_attn_fwd")
         return out
     code = _lib.lib().tj_attn_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],

@@ -69,6 +69,12 @@ int main() {
   expect("attn empty", tj_attn_fwd(nullptr, nullptr, nullptr, nullptr, TJ_F32, 0, 1, 16, 64, st, st, st, st, 0.125f, 1, nullptr, nullptr, nullptr, nullptr), TJ_OK);
   expect("attn bias alignment", tj_attn_fwd_proj_bias(q, k, v, o, TJ_F32, 1, 1, 16, 64, st, st, st, st, 0.125f, 1, nullptr, (const float*)at(4), nullptr, nullptr), TJ_ERR_ALIGN);
 
+  expect("attn small workspace", tj_attn_fwd_ws(q, k, v, o, TJ_F32, 1, 1, 8192, 64, st, st, st, st, 0.125f, 1, nullptr, nullptr, nullptr, nullptr, at(1024), 1024, nullptr), TJ_ERR_WORKSPACE);
+  expect("attn ws dtype", tj_attn_fwd_ws(q, k, v, o, 7, 1, 1, 8192, 64, st, st, st, st, 0.125f, 1, nullptr, nullptr, nullptr, nullptr, at(1024), 1024, nullptr), TJ_ERR_DTYPE);
+  expect_size("attn ws huge", tj_attn_workspace_bytes(kBig / 2, kBig / 2, kBig / 4, 64, 1), 0);
+  expect_size("attn ws many tiles", tj_attn_workspace_bytes(64, 16, 4096, 64, 1), 0);
+  expect_size("attn ws head dim", tj_attn_workspace_bytes(1, 1, 8192, 48, 1), 0);
+
   // workspace sizes: 0 for invalid or overflowing requests
   expect_size("poly ws invalid", tj_poly_workspace_bytes(0, 1, 4096, 64, 512), 0);
   expect_size("poly ws huge", tj_poly_workspace_bytes(kBig / 2, kBig / 2, 4096, 64, 512), 0);
