@@ -26,13 +26,25 @@ import torch
 
 def weights_signature(module: torch.nn.Module) -> tuple:
     """Addresses and in-place versions of every parameter and buffer."""
+    # Straight over the module dictionaries: parameters() and buffers() build
+    # names and sets on the way, several times the cost of the entries, and
+    # this runs before every replay.
     sig = []
-    for t in list(module.parameters()) + list(module.buffers()):
-        try:
-            version = t._version
-        except RuntimeError:  # inference tensors carry no version counter
-            version = None
-        sig.append((t.data_ptr(), version, tuple(t.shape), t.dtype))
+    stack = [module]
+    while stack:
+        m = stack.pop()
+        for tensors in (m._parameters, m._buffers):
+            for t in tensors.values():
+                if t is None:
+                    continue
+                try:
+                    version = t._version
+                except RuntimeError:  # inference tensors carry no version counter
+                    version = None
+                sig.append((t.data_ptr(), version, t.shape, t.dtype))
+        for sub in m._modules.values():
+            if sub is not None:
+                stack.append(sub)
     return tuple(sig)
 
 

@@ -11,7 +11,6 @@ without a host synchronisation. Tensors stay where they are: strided
 
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass
 from typing import Optional, Union
 
@@ -26,8 +25,10 @@ SUPPORTED_HEAD_DIMS = (32, 64, 128, 256)
 _DTYPES = {torch.float32: _lib.TJ_F32, torch.float16: _lib.TJ_F16}
 
 
-def _stream_ptr(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream_ptr(device: torch.device) -> int:
+    """The current stream of a tensor's device, without the Stream object
+    ``torch.cuda.current_stream`` builds."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -52,7 +53,7 @@ MAX_HEAD_SPAN_BYTES = 1 << 31
 
 
 def _head_span_bytes(t: torch.Tensor) -> int:
-    s, d = t.shape[2], t.shape[3]
+    _, _, s, d = t.shape
     return ((s - 1) * t.stride(2) + d) * t.element_size() if s > 0 else 0
 
 
@@ -67,10 +68,9 @@ def _kernel_view(t: torch.Tensor, keys: bool = False) -> torch.Tensor:
     (over 2^31 / (H*D*4) tokens in fp32) cost one copy instead of being
     refused.
     """
-    vec = 16 // t.element_size()
-    st = t.stride()
-    if (st[3] == 1 and all(s % vec == 0 for s in st[:3]) and t.data_ptr() % 16 == 0
-            and (not keys or (st[2] >= 0 and _head_span_bytes(t) < MAX_HEAD_SPAN_BYTES))):
+    sb, sh, ss, sd = t.stride()
+    if (sd == 1 and not (sb | sh | ss) & (16 // t.element_size() - 1) and not t.data_ptr() & 15
+            and (not keys or (ss >= 0 and _head_span_bytes(t) < MAX_HEAD_SPAN_BYTES))):
         return t
     return t.contiguous()
 
@@ -78,15 +78,16 @@ def _kernel_view(t: torch.Tensor, keys: bool = False) -> torch.Tensor:
 def _check_qkv(q, k, v):
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
         raise ValueError("q, k, v must be [B, H, S, D]")
-    if q.shape != k.shape or q.shape != v.shape:
+    shape = q.shape
+    if shape != k.shape or shape != v.shape:
         raise ValueError(f"q, k, v shapes differ: {tuple(q.shape)}, {tuple(k.shape)}, {tuple(v.shape)}")
     if q.dtype not in _DTYPES:
         raise UnsupportedCaseError(f"dtype {q.dtype} is not supported (float32 or float16)")
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError("q, k, v must share a dtype")
-    if kernel_head_dim(q.shape[-1]) is None:
+    if kernel_head_dim(shape[-1]) is None:
         raise UnsupportedCaseError(
-            f"head_dim {q.shape[-1]} is not supported (at most {SUPPORTED_HEAD_DIMS[-1]}; "
+            f"head_dim {shape[-1]} is not supported (at most {SUPPORTED_HEAD_DIMS[-1]}; "
             f"{SUPPORTED_HEAD_DIMS} natively, others zero-padded)"
         )
 
@@ -172,8 +173,10 @@ def scaled_dot_product_attention(
         qk_split = None
     for name, t, n in (("valid_len", valid_len, b), ("row_limit", row_limit, b * h),
                        ("qk_split", qk_split, b * h)):
-        if t is not None and (t.dtype != torch.int32 or t.device != dev or t.numel() != n
-                              or not t.is_contiguous()):
+        if t is None:
+            continue
+        if (t.dtype != torch.int32 or t.device != dev or t.numel() != n
+                or not t.is_contiguous()):
             raise ValueError(f"{name} must be a contiguous int32 tensor of {n} elements on {dev}")
     if q_bias is not None or v_bias is not None:
         if row_limit is not None or qk_split is not None:
@@ -186,7 +189,8 @@ def scaled_dot_product_attention(
     if row_limit is None:
         # Long sweeps over few query tiles are cut into parts, whose sums need
         # a workspace; 0 bytes for all other calls.
-        ws_bytes = _lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(bool(is_causal)))
+        # (never below 20 key tiles of 64, so short calls do not ask).
+        ws_bytes = _lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(bool(is_causal))) if s > 1216 else 0
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         code = _lib.lib().tj_attn_fwd_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],

@@ -37,8 +37,11 @@ def _check_out(out: Optional[torch.Tensor], x: torch.Tensor) -> None:
 
 
 def _ok(*ts: torch.Tensor) -> bool:
-    return all(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-               and t.shape[-1] % 4 == 0 for t in ts)
+    f32 = torch.float32
+    for t in ts:
+        if (t.dtype != f32 or not t.is_cuda or not t.is_contiguous() or t.data_ptr() & 15 or t.shape[-1] & 3):
+            return False
+    return True
 
 
 def bias_residual(x: torch.Tensor, y: torch.Tensor, bias: torch.Tensor, valid_len: Optional[torch.Tensor],

@@ -38,8 +38,11 @@ def _usable(x: torch.Tensor, *params: torch.Tensor) -> bool:
     if (not x.is_cuda or x.dtype != torch.float32 or torch.is_grad_enabled()
             or torch.get_float32_matmul_precision() == "highest" or not x.is_contiguous() or x.data_ptr() % 16):
         return False
-    return all(p is not None and p.dtype == torch.float32 and p.device == x.device and p.is_contiguous()
-               and p.data_ptr() % 16 == 0 for p in params)
+    dev = x.device
+    for p in params:
+        if (p is None or p.dtype != torch.float32 or p.device != dev or not p.is_contiguous() or p.data_ptr() % 16):
+            return False
+    return True
 
 
 def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional[torch.Tensor] = None,
@@ -47,15 +50,17 @@ def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional
     """``x @ w.T`` for up to three weights of one shape in one launch, or
     ``act(x @ w.T + bias)`` for one (``act`` "gelu" or "relu")."""
     n, k = weights[0].shape
-    m = x.numel() // k if k else 0
-    params = list(weights) + ([bias] if bias is not None else [])
-    if x.shape[-1] != k or m == 0 or not _usable(x, *params) or any(w.shape != (n, k) for w in weights):
-        return None
-    if n == NARROW and k == NARROW and act is None and m * n * k * len(weights) > ROWS_MAX_WORK:
-        narrow = 1
-    elif n % 32 == 0 and k % 64 == 0 and k <= ROWS_MAX_K and m * n * k * len(weights) <= ROWS_MAX_WORK:
+    if x.numel() * n * len(weights) <= ROWS_MAX_WORK:
+        if n & 31 or k & 63 or k > ROWS_MAX_K:
+            return None
         narrow = 0
+    elif n == NARROW and k == NARROW and act is None:
+        narrow = 1
     else:
+        return None
+    m = x.numel() // k
+    if (x.shape[-1] != k or m == 0 or not _usable(x, *weights, *(() if bias is None else (bias,)))
+            or any(w.shape != (n, k) for w in weights)):
         return None
     outs = [torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device) for _ in weights]
     ptrs = [w.data_ptr() for w in weights] + [None] * (3 - len(weights))

@@ -20,7 +20,6 @@ through these functions.
 
 from __future__ import annotations
 
-import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -30,10 +29,6 @@ from . import _lib
 from .attention import _require_device, _stream_ptr
 
 _W = 64  # head dim and value width of the kernels
-
-
-def _strides3(t: torch.Tensor) -> ctypes.Array:
-    return (ctypes.c_int64 * 3)(*t.stride())
 
 
 def _half_rows(t: torch.Tensor) -> torch.Tensor:
@@ -87,7 +82,7 @@ def quad_apply(a: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
     code = _lib.lib().tj_quad_apply(
         a16.data_ptr(), sp.data_ptr(), y.data_ptr(),
         _lib.TJ_F32 if sp.dtype == torch.float32 else _lib.TJ_F16,
-        m, c, _W, _W, _strides3(a16), _strides3(sp), _strides3(y), _stream_ptr(dev),
+        m, c, _W, _W, _lib.strides3(a16), _lib.strides3(sp), _lib.strides3(y), _stream_ptr(dev),
     )
     _lib.check(code, "tj_quad_apply")
     return y[..., :vw].to(a.dtype)
@@ -124,15 +119,15 @@ def quad_update(
                                       and shadow.stride(1) % 8 == 0 and shadow.data_ptr() % 16 == 0)):
         code = _lib.lib().tj_quad_update(
             b16.data_ptr(), v16.data_ptr(), out.data_ptr(), None if shadow is None else shadow.data_ptr(),
-            m, c, _W, _W, _strides3(b16), _strides3(v16), _strides3(out),
-            None if shadow is None else _strides3(shadow), _stream_ptr(dev),
+            m, c, _W, _W, _lib.strides3(b16), _lib.strides3(v16), _lib.strides3(out),
+            None if shadow is None else _lib.strides3(shadow), _stream_ptr(dev),
         )
         _lib.check(code, "tj_quad_update")
         return
     delta = torch.zeros(m, _W * _W, _W, dtype=torch.float32, device=dev)
     code = _lib.lib().tj_quad_update(
         b16.data_ptr(), v16.data_ptr(), delta.data_ptr(), None,
-        m, c, _W, _W, _strides3(b16), _strides3(v16), _strides3(delta), None, _stream_ptr(dev),
+        m, c, _W, _W, _lib.strides3(b16), _lib.strides3(v16), _lib.strides3(delta), None, _stream_ptr(dev),
     )
     _lib.check(code, "tj_quad_update")
     out += delta.reshape(m, _W, _W, _W)[:, :d, :d, :vw].reshape(m, d * d, vw)
@@ -157,7 +152,7 @@ def causal_diag(a: torch.Tensor, b: torch.Tensor, v: torch.Tensor) -> Tuple[torc
     den = torch.empty(m, c, dtype=torch.float32, device=dev)
     code = _lib.lib().tj_causal_diag(
         a16.data_ptr(), b16.data_ptr(), v16.data_ptr(), num.data_ptr(), den.data_ptr(),
-        m, c, _W, _W, _strides3(a16), _strides3(b16), _strides3(v16), _strides3(num), den.stride(0),
+        m, c, _W, _W, _lib.strides3(a16), _lib.strides3(b16), _lib.strides3(v16), _lib.strides3(num), den.stride(0),
         _stream_ptr(dev),
     )
     _lib.check(code, "tj_causal_diag")
