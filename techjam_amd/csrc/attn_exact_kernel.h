@@ -251,6 +251,10 @@ struct KVStage {
   }
 };
 
+// A part's row sum is zero exactly where it has no keys for the row. Tested by
+// bits: NaN sums count as keys, and this file is built without NaN comparisons.
+__device__ __forceinline__ bool has_keys(float sum) { return (__builtin_bit_cast(uint32_t, sum) << 1) != 0; }
+
 // One query tile of one (b, h): 4 waves x 32*QB rows. Each wave holds QB
 // 32-row query blocks, so every K / V^T operand read from LDS feeds QB MFMAs.
 // SPLIT selects the three-MFMA score path.
@@ -412,6 +416,11 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
         // by more than 2^8 (p <= 256 is exact enough in fp16 and harmless in the
         // fp32 accumulators); the first tile always sets it.
         shift[qb] = first ? t_max : (t_max > kRescaleLog2 ? t_max : 0.f);
+        // A later part may start on keys that all score -inf (k beyond fp16):
+        // they weigh nothing, as in a sweep that started before them.
+        if constexpr (PART) {
+          if (kt0 > 0 && first && t_max == -__builtin_inff()) shift[qb] = 0.f;
+        }
       }
       // One wave-wide decision per tile for all query blocks (a lane or block
       // whose shift is 0 rescales by exactly 1).
@@ -509,8 +518,9 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
             *reinterpret_cast<float4_t*>(po + db * 32 + 8 * g + 4 * hl) =
                 float4_t{oacc[qb][db][4 * g], oacc[qb][db][4 * g + 1], oacc[qb][db][4 * g + 2], oacc[qb][db][4 * g + 3]};
         if (hl == 0) {
-          // A wave without keys in this part leaves sum 0; its reference is not read.
-          a.part_ml[(slot * 128 + row) * 2] = l_tot > 0.f ? m_run[qb] : 0.f;
+          // A wave without keys in this part leaves sum 0; its reference is not
+          // read. A NaN sum goes on as it is.
+          a.part_ml[(slot * 128 + row) * 2] = has_keys(l_tot) ? m_run[qb] : 0.f;
           a.part_ml[(slot * 128 + row) * 2 + 1] = l_tot;
         }
         continue;
@@ -722,21 +732,22 @@ __global__ __launch_bounds__(NT) void combine_parts_kernel(AttnArgs a) {
 #pragma unroll 8
     for (int p = 0; p < np; ++p) {
       const float2_t x = ml[p * 128];
-      m = x[1] > 0.f ? fmaxf(m, x[0]) : m;
+      m = has_keys(x[1]) ? fmaxf(m, x[0]) : m;
     }
     float l = 0.f;
 #pragma unroll 4
     for (int p = 0; p < np; ++p) {
       const float2_t x = ml[p * 128];
       const float4_t o = *reinterpret_cast<const float4_t*>(po + (int64_t)p * 128 * HD);
-      const float wgt = x[1] > 0.f ? fast_exp2(x[0] - m) : 0.f;  // a part without keys holds zeros
+      const float wgt = has_keys(x[1]) ? fast_exp2(x[0] - m) : 0.f;  // a part without keys holds zeros
       l += wgt * x[1];
       y += wgt * o;
     }
     const float4_t bv = a.v_bias != nullptr ? *reinterpret_cast<const float4_t*>(a.v_bias + h * HD + c) : float4_t{0.f, 0.f, 0.f, 0.f};
-    const float inv = 1.f / l;
+    const bool live = l > 0.f;
+    const float inv = live ? 1.f / l : 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = l > 0.f ? y[e] * inv + bv[e] : 0.f;
+    for (int e = 0; e < 4; ++e) y[e] = y[e] * inv + (live ? bv[e] : 0.f);  // NaN stays NaN, as in one sweep
   }
   T* op = reinterpret_cast<T*>(a.o) + a.vo.row(b, h, qi) + c;
   if constexpr (sizeof(T) == 4) *reinterpret_cast<float4_t*>(op) = y;

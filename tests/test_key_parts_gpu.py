@@ -110,3 +110,28 @@ def test_capture_replays_with_the_parts(cuda):
         torch.cuda.synchronize()
         assert torch.equal(got, want)
         torch.randn(1 << 20, device=cuda).sum().item()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_nan_and_infinite_keys_as_in_one_sweep(cuda, causal, dtype):
+    """A row that sees a NaN score is NaN whatever its other parts hold; keys
+    that all score -inf weigh nothing, also where a part starts on them."""
+    from techjam_amd.kernels import _lib, scaled_dot_product_attention
+
+    b, h, s, d = 1, 2, 4096, 64
+    assert _lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(causal)) > 0
+    g = torch.Generator(device=cuda).manual_seed(11)
+    q, k, v = (torch.randn(b, s, h, d, generator=g, device=cuda).to(dtype).transpose(1, 2) for _ in range(3))
+    q[0, 1, :, 0] = q[0, 1, :, 0].abs() + 0.5
+    k[0, 0, 2000, 3] = float("nan")
+    for t0 in range(512, s, 512):  # whole key tiles at every possible start of a part
+        k[0, 1, t0:t0 + 64, 0] = -float("inf")
+    got = scaled_dot_product_attention(q, k, v, is_causal=causal)
+    want = _one_sweep(q, k, v, causal, None, None, None)
+    torch.cuda.synchronize()
+    bad = torch.isnan(want).any(-1)
+    assert bool(bad[0, 0, -1]) and not bool(bad[0, 1].any())
+    assert torch.equal(torch.isnan(got).any(-1), bad)
+    tol = 2 * 2 ** -11 * float(v.abs().max()) + (2 ** -10 * float(v.abs().max()) if dtype == torch.float16 else 1e-5)
+    assert float((got - want)[~bad].abs().max()) <= tol
