@@ -97,19 +97,22 @@ def test_split_scores_in_parts(cuda, d, dtype):
 def test_capture_replays_with_the_parts(cuda):
     from techjam_amd.kernels import scaled_dot_product_attention
 
-    g = torch.Generator(device=cuda).manual_seed(5)
-    q, k, v = (torch.randn(1, 4096, 2, 64, generator=g, device=cuda).transpose(1, 2) for _ in range(3))
-    want = scaled_dot_product_attention(q, k, v, is_causal=True)
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        got = scaled_dot_product_attention(q, k, v, is_causal=True)
-    for _ in range(3):
-        got.zero_()
-        graph.replay()
+    # Inference mode throughout: a capture earlier in the process leaves its
+    # random state as an inference tensor.
+    with torch.inference_mode():
+        g = torch.Generator(device=cuda).manual_seed(5)
+        q, k, v = (torch.randn(1, 4096, 2, 64, generator=g, device=cuda).transpose(1, 2) for _ in range(3))
+        want = scaled_dot_product_attention(q, k, v, is_causal=True)
         torch.cuda.synchronize()
-        assert torch.equal(got, want)
-        torch.randn(1 << 20, device=cuda).sum().item()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = scaled_dot_product_attention(q, k, v, is_causal=True)
+        for _ in range(3):
+            got.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+            torch.randn(1 << 20, device=cuda).sum().item()
 
 
 @pytest.mark.parametrize("causal", [True, False])
