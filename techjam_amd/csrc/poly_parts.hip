@@ -28,6 +28,8 @@ constexpr int XT = 256;       // threads per workgroup
 constexpr int XLP = 72;       // padded LDS row (144 bytes)
 constexpr int XAP = 66;       // padded row of the a tile (132 bytes)
 
+using float2_t = float __attribute__((ext_vector_type(2)));
+
 struct View3 {
   int64_t sm, sr;  // strides of the outer two dims (elements); innermost is 1
   __device__ __forceinline__ int64_t at(int m, int r) const { return (int64_t)m * sm + (int64_t)r * sr; }
@@ -58,6 +60,15 @@ struct HalfTile {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       *reinterpret_cast<half4_t*>(&dst[4 * c + e][4 * g]) = half4_t{x[0][e], x[1][e], x[2][e], x[3][e]};
+  }
+  // The same with the even dims in the first half of the rows and the odd
+  // ones in the second: dim 2 x + e at row 32 e + x.
+  __device__ __forceinline__ void store_t_pairs(half_t (*dst)[XLP], int tid) const {
+    int g, c;
+    coords(tid, g, c);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      *reinterpret_cast<half4_t*>(&dst[32 * (e & 1) + 2 * c + (e >> 1)][4 * g]) = half4_t{x[0][e], x[1][e], x[2][e], x[3][e]};
   }
   // [row][dim].
   __device__ __forceinline__ void store_rows(half_t (*dst)[XLP], int tid) const {
@@ -110,7 +121,7 @@ struct ApplyArgs {
 // for the MFMA A operand -- so a load in flight holds no conversion back.
 template <typename TS>
 struct HalfSlice {
-  using Raw = std::conditional_t<sizeof(TS) == 4, float __attribute__((ext_vector_type(2))), half2_t>;
+  using Raw = std::conditional_t<sizeof(TS) == 4, float2_t, half2_t>;
   Raw x[4];
   // This thread's first element of slice 0: row 4 g, column 32 vh + 2 c of S[m].
   __device__ __forceinline__ static const TS* origin(const TS* s, const View3& vs, int m, int vh, int tid) {
@@ -255,7 +266,10 @@ struct UpdateArgs {
 // v of the head from HBM (2x the algorithmic fetch), but the state traffic
 // spreads more evenly and the launch runs ~5 % faster than with the 16
 // workgroups of one m kept on one XCD.
-// acc[jb][vb] holds D[j][v] of S_i, i.e. state rows i*64 + j, columns v.
+// acc[jb][vb] holds D[j][v] of S_i, i.e. state rows i*64 + j, column 2 ln + vb:
+// v^T is staged even columns first (store_t_pairs), so that a lane's two
+// blocks are neighbouring columns and the state is read and written 8 bytes
+// (its shadow 4 bytes) a lane, whole rows an instruction.
 __global__ __launch_bounds__(XT, 2) void quad_update_kernel(UpdateArgs a) {
   __shared__ half_t bt[2][XD][XLP];
   __shared__ half_t vt[2][XD][XLP];
@@ -265,16 +279,16 @@ __global__ __launch_bounds__(XT, 2) void quad_update_kernel(UpdateArgs a) {
 
   float16_t acc[2][2];
   {
-    const float* base = a.s + a.vs.at(m, i * XD) + ln;
+    const float* base = a.s + a.vs.at(m, i * XD) + 2 * ln;
 #pragma unroll
     for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
-      for (int vb = 0; vb < 2; ++vb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = 32 * jb + 8 * (r / 4) + 4 * hl + (r % 4);
-          acc[jb][vb][r] = base[(int64_t)j * a.vs.sr + 32 * vb];
-        }
+      for (int r = 0; r < 16; ++r) {
+        const int j = 32 * jb + 8 * (r / 4) + 4 * hl + (r % 4);
+        const float2_t x = *reinterpret_cast<const float2_t*>(base + (int64_t)j * a.vs.sr);
+        acc[jb][0][r] = x[0];
+        acc[jb][1][r] = x[1];
+      }
   }
 
   const int n_blk = (a.C + 63) / 64;
@@ -283,7 +297,7 @@ __global__ __launch_bounds__(XT, 2) void quad_update_kernel(UpdateArgs a) {
     tb.load(a.b, a.vb, m, 0, a.C, tid);
     tv.load(a.v, a.vv, m, 0, a.C, tid);
     tb.store_t(bt[0], tid);
-    tv.store_t(vt[0], tid);
+    tv.store_t_pairs(vt[0], tid);
   }
   __syncthreads();
   for (int blk = 0; blk < n_blk; ++blk) {
@@ -311,24 +325,23 @@ __global__ __launch_bounds__(XT, 2) void quad_update_kernel(UpdateArgs a) {
     }
     if (blk + 1 < n_blk) {
       tb.store_t(bt[cur ^ 1], tid);
-      tv.store_t(vt[cur ^ 1], tid);
+      tv.store_t_pairs(vt[cur ^ 1], tid);
     }
     __syncthreads();
   }
 
-  float* sbase = a.s + a.vs.at(m, i * XD) + ln;
-  half_t* hbase = a.shadow != nullptr ? a.shadow + a.vsh.at(m, i * XD) + ln : nullptr;
+  float* sbase = a.s + a.vs.at(m, i * XD) + 2 * ln;
+  half_t* hbase = a.shadow != nullptr ? a.shadow + a.vsh.at(m, i * XD) + 2 * ln : nullptr;
 #pragma unroll
   for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
-    for (int vb = 0; vb < 2; ++vb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int j = 32 * jb + 8 * (r / 4) + 4 * hl + (r % 4);
-        const float x = acc[jb][vb][r];
-        sbase[(int64_t)j * a.vs.sr + 32 * vb] = x;
-        if (hbase != nullptr) hbase[(int64_t)j * a.vsh.sr + 32 * vb] = (half_t)x;
-      }
+    for (int r = 0; r < 16; ++r) {
+      const int j = 32 * jb + 8 * (r / 4) + 4 * hl + (r % 4);
+      const float2_t x = {acc[jb][0][r], acc[jb][1][r]};
+      *reinterpret_cast<float2_t*>(sbase + (int64_t)j * a.vs.sr) = x;
+      if (hbase != nullptr)
+        *reinterpret_cast<half2_t*>(hbase + (int64_t)j * a.vsh.sr) = half2_t{(half_t)x[0], (half_t)x[1]};
+    }
 }
 
 // ---------------------------------------------------------------------------
