@@ -88,6 +88,14 @@ struct HalfTile {
   }
 };
 
+// Orders a wave's own LDS writes and reads across its lanes: the LDS serves one
+// wave in order, so only the compiler has to be kept from reordering them.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // a tile of one 128-row block: B operands (dims 16 ks + 8 hl .. +7 of row
 // c0 + 32 w + ln) and the a tile in LDS for the per-i scalars.
 __device__ __forceinline__ void load_a_rows(const half_t* a, const View3& va, int m, int c0, int C,
@@ -440,6 +448,124 @@ __global__ __launch_bounds__(XT, 2) void causal_diag_kernel(DiagArgs a) {
   if (hl == 0) a.den[(int64_t)m * a.den_sm + qi] = den;
 }
 
+// The same where 128-row blocks leave the chip idle: one workgroup per (m, 32
+// rows), whose four waves take the 32-key blocks up to the rows' own in turn
+// (wave w blocks w, w + 4, ..), each with its keys straight from global memory
+// and its own V^T tile in LDS, so the sweep has no barrier, and their sums are
+// added through LDS at the end. The exp and conversion of each weight bound it
+// (about 40 VALU cycles against 16 of MFMA), so what counts is that every SIMD
+// gets its share of the pairs; the price is that K and V are loaded, and V
+// transposed, once per 32 rows. Kernel us, 128-row blocks / here: 32 m x 512
+// rows 13.8 / 10.2, 32 x 100 6.1 / 4.3, 8 x 2048 39.9 / 26.0, 4 x 4096 76.0 /
+// 46.0, 1 x 8192 147.5 / 57.2. By the number of 128-row blocks, 384 of them
+// 21.3 / 20.3, 512 22.4 / 25.4 (128 x 512) and 64.8 / 68.8 (32 x 2048), 1024
+// 37.4 / 45.3: two such blocks on every CU keep it busy, and the line is there.
+constexpr int64_t kDiagWide = 512;
+constexpr int DKP = 40;      // padded row of a V^T tile (80 bytes: 16 rows hit 16 distinct 16-byte slots)
+constexpr int DRP = XD + 4;  // padded row of the partial sums
+
+__global__ __launch_bounds__(XT, 2) void causal_diag_blocks_kernel(DiagArgs a) {
+  constexpr int NW = XT / kWave;
+  __shared__ __attribute__((aligned(16))) union {
+    half_t vt[NW][XD][DKP];
+    float part[NW][32][DRP];
+  } sm;
+  __shared__ float dpart[NW][32];
+  const int n_rb = (a.C + 31) / 32;
+  const int m = blockIdx.x, rb = n_rb - 1 - blockIdx.y;  // longest sweeps first
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave, hl = lane / 32, ln = lane % 32;
+  const int c0 = 32 * rb;
+
+  half8_t aB[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    aB[ks] = c0 + ln < a.C ? *reinterpret_cast<const half8_t*>(a.a + a.va.at(m, c0 + ln) + 16 * ks + 8 * hl)
+                           : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+
+  // Score row ln is the block's key ln with bits 2 and 3 swapped: accumulator
+  // element r then holds key 16 (r / 8) + 8 hl + r % 8, and eight consecutive
+  // ones are a k-step's operand. Keys past C, all above the diagonal, repeat
+  // the last.
+  const int kr = (ln & 19) | ((ln & 4) << 1) | ((ln & 8) >> 1), vg = lane & 7, vc = lane >> 3;
+  half8_t kx[4], vx[4];
+  auto load = [&](int kb) {
+    const half_t* kp = a.b + a.vb.at(m, min(32 * kb + kr, a.C - 1)) + 8 * hl;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) kx[ks] = *reinterpret_cast<const half8_t*>(kp + 16 * ks);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      vx[r] = *reinterpret_cast<const half8_t*>(a.v + a.vv.at(m, min(32 * kb + 4 * vg + r, a.C - 1)) + 8 * vc);
+  };
+
+  float16_t accd[2];
+#pragma unroll
+  for (int vb = 0; vb < 2; ++vb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) accd[vb][r] = 0.f;
+  float den = 0.f, den2 = 0.f;
+
+  if (w <= rb) load(w);
+  for (int kb = w; kb <= rb; kb += NW) {
+    float16_t sc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) sc = mfma32(kx[ks], aB[ks], sc);
+    wave_lds_order();  // the tile's earlier reads stay before these writes
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      *reinterpret_cast<half4_t*>(&sm.vt[w][8 * vc + e][4 * vg]) = half4_t{vx[0][e], vx[1][e], vx[2][e], vx[3][e]};
+    wave_lds_order();  // and the writes of all lanes before the reads below
+    if (kb + NW <= rb) load(kb + NW);
+    half8_t pf[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) pf[r / 8][r % 8] = (half_t)fast_exp2(sc[r] * 1.4426950408889634f);
+    if (kb == rb) {  // the diagonal block
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (16 * (r / 8) + 8 * hl + r % 8 > ln) pf[r / 8][r % 8] = (half_t)0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      den += (float)pf[0][r];
+      den2 += (float)pf[1][r];
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int vb = 0; vb < 2; ++vb)
+        accd[vb] = mfma32(*reinterpret_cast<const half8_t*>(&sm.vt[w][32 * vb + ln][16 * x + 8 * hl]), pf[x], accd[vb]);
+  }
+  den = pair_sum(den + den2);
+
+  __syncthreads();  // every wave is done with its V^T tile
+#pragma unroll
+  for (int vb = 0; vb < 2; ++vb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<float4_t*>(&sm.part[w][ln][32 * vb + 8 * g + 4 * hl]) =
+          float4_t{accd[vb][4 * g], accd[vb][4 * g + 1], accd[vb][4 * g + 2], accd[vb][4 * g + 3]};
+  if (hl == 0) dpart[w][ln] = den;
+  __syncthreads();
+  const int row = tid / 8, v0 = 8 * (tid % 8);
+  if (c0 + row < a.C) {
+    float* np = a.num + a.vn.at(m, c0 + row) + v0;
+#pragma unroll
+    for (int x = 0; x < 8; x += 4) {
+      float4_t y = *reinterpret_cast<const float4_t*>(&sm.part[0][row][v0 + x]);
+#pragma unroll
+      for (int p = 1; p < NW; ++p) y += *reinterpret_cast<const float4_t*>(&sm.part[p][row][v0 + x]);
+      *reinterpret_cast<float4_t*>(np + x) = y;
+    }
+    if (v0 == 0) {
+      float d = dpart[0][row];
+#pragma unroll
+      for (int p = 1; p < NW; ++p) d += dpart[p][row];
+      a.den[(int64_t)m * a.den_sm + c0 + row] = d;
+    }
+  }
+}
+
 bool view3_ok(const void* p, const int64_t st[3], int elt) {
   if (p == nullptr || st == nullptr || st[2] != 1 || !tjh::aligned16(p)) return false;
   const int64_t vec = 16 / elt;
@@ -527,7 +653,11 @@ extern "C" int tj_causal_diag(const void* a, const void* b, const void* v, float
   args.den_sm = den_stride_m;
   args.M = (int)M;
   args.C = (int)C;
-  hipLaunchKernelGGL(tj::causal_diag_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)M), dim3(tj::XT), 0,
-                     stream, args);
+  if ((C + 127) / 128 * M < tj::kDiagWide) {
+    // m fastest: with M a multiple of 8, one m's workgroups share an XCD's L2.
+    hipLaunchKernelGGL(tj::causal_diag_blocks_kernel, dim3((unsigned)M, (unsigned)((C + 31) / 32)), dim3(tj::XT), 0, stream, args);
+  } else {
+    hipLaunchKernelGGL(tj::causal_diag_kernel, dim3((unsigned)((C + 127) / 128), (unsigned)M), dim3(tj::XT), 0, stream, args);
+  }
   return tjh::launch_status();
 }
