@@ -26,7 +26,7 @@
 //     reads two [tokens, 128] tensors and writes two. Bound by HBM for many
 //     tokens: at 65 536 (26 us for its bytes at the copy rate) the q, k, v
 //     projections take 40 us (52 as three library products), out_proj +
-//     residual + norm 31 (38), the FFN half 46 (66).
+//     residual + norm 31 (38), the FFN half 41 (66; 49 with erff in its GELU).
 #include "tj_common.h"
 
 namespace tj {
@@ -65,7 +65,7 @@ __device__ __forceinline__ float8_t load8(const float* p) {
 
 template <Act A>
 __device__ __forceinline__ float activate(float t) {
-  if constexpr (A == ACT_GELU) return 0.5f * t * (1.f + erff(t * 0.70710678118654752f));
+  if constexpr (A == ACT_GELU) return gelu_erf(t);
   else if constexpr (A == ACT_RELU) return t > 0.f ? t : 0.f;
   else return t;
 }
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(NT, KIND == NARROW_FFN ? 1 : 2) void narrow_kernel(
       // k-slots of step 2 nb + x in the key_slot order W2 is staged in.
 #pragma unroll
       for (int nb = 0; nb < 4; ++nb) {
-        __builtin_amdgcn_sched_barrier(0);  // one block's erf temporaries at a time
+        __builtin_amdgcn_sched_barrier(0);  // one block's temporaries at a time
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const float4_t b = *reinterpret_cast<const float4_t*>(a.bias_in + 32 * nb + 8 * g + 4 * hl);

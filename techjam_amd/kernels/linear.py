@@ -29,7 +29,7 @@ ROWS_MAX_K = 512
 #: Tokens from which the one-pass kernels beat a product and the passes after
 #: it, and up to which the shorter one does (us, library + passes / here:
 #: residual + norm 16 384 tokens 16.4 / 16.4, 65 536 38 / 31, 262 144 146 / 155;
-#: FFN 30 / 38, 66 / 46, 249 / 205): below, one tile's latency is all there is.
+#: FFN 30 / 38, 66 / 41, 249 / 205): below, one tile's latency is all there is.
 NARROW_MIN_TOKENS = 24576
 NARROW_RESIDUAL_MAX_TOKENS = 131072
 
