@@ -56,7 +56,12 @@ __device__ __forceinline__ float gelu_erf(float x) {
   p = fmaf(p, t, -0.4592081904411316f);
   p = fmaf(p, t, -1.1511051654815674f);
   const float e = fast_exp2(p * t);
-  return fmaf(-0.5f * fabsf(fminf(x, 1e30f)), e, fmaxf(x, 0.f));
+  float y = fmaf(-0.5f * fabsf(fminf(x, 1e30f)), e, fmaxf(x, 0.f));
+  // The fp32 value, also for a caller that rounds it to fp16: free to, the
+  // compiler fuses the two roundings (v_fma_mixlo_f16), and the fp16 outputs
+  // would not be the fp32 ones rounded.
+  asm("" : "+v"(y));
+  return y;
 }
 
 // Workgroup barrier without the memory fences of __syncthreads() (which also
