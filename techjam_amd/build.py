@@ -50,6 +50,7 @@ FLAGS = [
 # strategy (faster for it; the default scheduler is faster for the others).
 FILE_FLAGS = {
     "attn_exact.hip": ["-fno-honor-nans"],
+    "attn_exact_parts.hip": ["-fno-honor-nans"],
     "attn_exact_split.hip": ["-fno-honor-nans", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
 }
 

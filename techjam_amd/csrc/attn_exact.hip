@@ -73,16 +73,6 @@ PartPlan plan_parts(int64_t B, int64_t H, int64_t S, int64_t D, int causal) {
 }
 
 template <typename T>
-int dispatch_parts(const AttnArgs& a, int64_t D, hipStream_t stream) {
-  switch (D) {
-    case 32: return launch_parts<T, 32>(a, stream);
-    case 64: return launch_parts<T, 64>(a, stream);
-    case 128: return launch_parts<T, 128>(a, stream);
-    default: return launch_parts<T, 256>(a, stream);
-  }
-}
-
-template <typename T>
 int dispatch_hd(const AttnArgs& a, int64_t D, hipStream_t stream) {
   switch (D) {
     case 32: return launch<T, 32>(a, stream);
@@ -141,7 +131,7 @@ int attn_fwd(const void* q, const void* k, const void* v, void* o, int dtype, in
     a.n_mtiles = plan.n_mtiles;
     a.part_o = static_cast<float*>(workspace);
     a.part_ml = a.part_o + B * H * plan.n_parts * 128 * D;
-    return dtype == TJ_F32 ? tj::dispatch_parts<float>(a, D, stream) : tj::dispatch_parts<half_t>(a, D, stream);
+    return dtype == TJ_F32 ? tj::dispatch_parts_f32(a, D, stream) : tj::dispatch_parts_f16(a, D, stream);
   }
   if (dtype == TJ_F32) return tj::dispatch_hd<float>(a, D, stream);
   return tj::dispatch_hd<half_t>(a, D, stream);

@@ -86,6 +86,10 @@ struct AttnArgs {
 // (fp32 inputs, head_dim 64), built in attn_exact_split.hip.
 int launch_split_wide(const AttnArgs& a, hipStream_t stream);
 
+// The key parts (attn_exact_parts.hip).
+int dispatch_parts_f32(const AttnArgs& a, int64_t D, hipStream_t stream);
+int dispatch_parts_f16(const AttnArgs& a, int64_t D, hipStream_t stream);
+
 namespace {
 
 constexpr int BN = 64;     // keys per tile (kernels take a tile width BNT: 64, or 32)
