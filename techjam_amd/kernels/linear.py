@@ -1,12 +1,11 @@
 """Dense layers of the encoder block on the split-bf16 HIP kernels.
 
-They do the arithmetic of the GEMM library's fast float32 mode (operands
-split into two bf16 parts, three products, fp32 accumulation; same error
-against 64 bits), so they are used only where a caller allows that mode
-(``torch.get_float32_matmul_precision() != "highest"``) and, as a raw kernel
-call records no graph, only while gradients are off. Each function returns
-``None`` for what it does not take or is not faster at, and the caller then
-uses the library.
+They do the arithmetic of hipBLASLt's fast float32 mode (operands split into
+two bf16 parts, three products, fp32 accumulation; same error against 64
+bits), so they are used only where a float32 product would run in that mode
+(:func:`fast_float32_matmul`) and, as a raw kernel call records no graph, only
+while gradients are off. Each function returns ``None`` for what it does not
+take or is not faster at, and the caller then uses the library.
 """
 
 from __future__ import annotations
@@ -34,9 +33,31 @@ NARROW_MIN_TOKENS = 24576
 NARROW_RESIDUAL_MAX_TOKENS = 131072
 
 
+#: The setting float32 GEMMs on the GPU obey (``torch.backends.cuda.matmul.
+#: fp32_precision``, at a third of that property's cost); ``None`` on a torch
+#: without it.
+_fp32_precision = getattr(torch._C, "_get_fp32_precision_getter", None)
+
+
+def fast_float32_matmul() -> bool:
+    """Whether a float32 product on the GPU runs on split bf16 operands.
+
+    That is hipBLASLt's fast mode: the other BLAS backends compute in plain
+    float32 at any setting (256 x 256 x 256: 2.9e-7 of error, split 4.4e-6).
+    ``torch.get_float32_matmul_precision()`` does not tell -- it still says
+    "high" after ``torch.backends.cuda.matmul.fp32_precision`` was set to
+    "ieee", and raises where the two disagree the other way.
+    """
+    if _fp32_precision is None:
+        fast = torch.get_float32_matmul_precision() != "highest"
+    else:
+        fast = _fp32_precision("cuda", "matmul") == "tf32"
+    return fast and torch._C._get_blas_preferred_backend() == torch._C._BlasBackend.Cublaslt
+
+
 def _usable(x: torch.Tensor, *params: torch.Tensor) -> bool:
     if (not x.is_cuda or x.dtype != torch.float32 or torch.is_grad_enabled()
-            or torch.get_float32_matmul_precision() == "highest" or not x.is_contiguous() or x.data_ptr() % 16):
+            or not fast_float32_matmul() or not x.is_contiguous() or x.data_ptr() % 16):
         return False
     dev = x.device
     for p in params:

@@ -1,0 +1,42 @@
+"""When the split-bf16 dense layers may stand in for a float32 product (CPU):
+exactly where the product itself would run in hipBLASLt's fast mode."""
+
+from __future__ import annotations
+
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+# A process of its own: the settings are global and cannot all be set back.
+_PROBE = """
+import sys, types, torch
+from techjam_amd.kernels.linear import _usable
+x = types.SimpleNamespace(is_cuda=True, dtype=torch.float32, device=torch.device("cuda", 0),
+                          is_contiguous=lambda: True, data_ptr=lambda: 0)
+mm = torch.backends.cuda.matmul
+exec(sys.argv[1])
+with torch.no_grad():
+    print(_usable(x))
+"""
+
+
+@pytest.mark.parametrize("settings,usable", [
+    ("", False),
+    ("torch.set_float32_matmul_precision('high')", True),
+    ("torch.set_float32_matmul_precision('medium')", True),
+    ("mm.allow_tf32 = True", True),
+    ("mm.fp32_precision = 'tf32'", True),
+    ("torch.backends.fp32_precision = 'tf32'", True),
+    ("torch.set_float32_matmul_precision('highest')", False),
+    ("torch.set_float32_matmul_precision('high'); mm.fp32_precision = 'ieee'", False),
+    ("torch.set_float32_matmul_precision('high'); mm.allow_tf32 = False", False),
+    ("torch.set_float32_matmul_precision('high'); torch.backends.cuda.preferred_blas_library('cublas')", False),
+])
+def test_the_setting_the_gemms_obey_decides(settings, usable):
+    res = subprocess.run([sys.executable, "-c", _PROBE, settings], capture_output=True, text=True, cwd=ROOT, timeout=300)
+    assert res.returncode == 0, res.stderr[-2000:]
+    assert res.stdout.strip() == str(usable)
