@@ -81,8 +81,8 @@ def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional
         return None
     m = x.numel() // k
     if (x.shape[-1] != k or m == 0 or not _usable(x, *weights, *(() if bias is None else (bias,)))
-            or any(w.shape != (n, k) for w in weights)):
-        return None
+            or any(w.shape != (n, k) for w in weights) or (bias is not None and bias.shape != (n,))):
+        return None  # the kernel reads n values of the bias
     outs = [torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device) for _ in weights]
     ptrs = [w.data_ptr() for w in weights] + [None] * (3 - len(weights))
     optr = [o.data_ptr() for o in outs] + [None] * (3 - len(weights))

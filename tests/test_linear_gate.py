@@ -8,6 +8,7 @@ import sys
 from pathlib import Path
 
 import pytest
+import torch
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -40,3 +41,14 @@ def test_the_setting_the_gemms_obey_decides(settings, usable):
     res = subprocess.run([sys.executable, "-c", _PROBE, settings], capture_output=True, text=True, cwd=ROOT, timeout=300)
     assert res.returncode == 0, res.stderr[-2000:]
     assert res.stdout.strip() == str(usable)
+
+
+@pytest.mark.parametrize("size", [(32,), (1,), (128,), (1, 64)])
+def test_a_bias_of_another_size_stays_off_the_kernel(monkeypatch, size):
+    """The kernel reads as many bias values as the weight has rows."""
+    from techjam_amd.kernels import linear
+
+    monkeypatch.setattr(linear, "_usable", lambda *t: True)
+    monkeypatch.setattr(linear._lib, "lib", lambda: pytest.fail("the kernel would be called"))
+    x, w = torch.zeros(4, 128), torch.zeros(64, 128)
+    assert linear.projections(x, (w,), torch.zeros(size), "gelu") is None
