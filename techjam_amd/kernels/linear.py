@@ -57,7 +57,8 @@ def fast_float32_matmul() -> bool:
 
 def _usable(x: torch.Tensor, *params: torch.Tensor) -> bool:
     if (not x.is_cuda or x.dtype != torch.float32 or torch.is_grad_enabled()
-            or not fast_float32_matmul() or not x.is_contiguous() or x.data_ptr() % 16):
+            or not fast_float32_matmul() or not x.is_contiguous() or x.data_ptr() % 16
+            or torch.is_autocast_enabled("cuda")):  # the product would give the autocast type
         return False
     dev = x.device
     for p in params:

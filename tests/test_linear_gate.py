@@ -36,6 +36,7 @@ with torch.no_grad():
     ("torch.set_float32_matmul_precision('high'); mm.fp32_precision = 'ieee'", False),
     ("torch.set_float32_matmul_precision('high'); mm.allow_tf32 = False", False),
     ("torch.set_float32_matmul_precision('high'); torch.backends.cuda.preferred_blas_library('cublas')", False),
+    ("torch.set_float32_matmul_precision('high'); torch.set_autocast_enabled('cuda', True)", False),
 ])
 def test_the_setting_the_gemms_obey_decides(settings, usable):
     res = subprocess.run([sys.executable, "-c", _PROBE, settings], capture_output=True, text=True, cwd=ROOT, timeout=300)
