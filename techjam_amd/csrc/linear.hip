@@ -25,7 +25,7 @@
 //     place into the second product's operand: the whole FFN half of a block
 //     reads two [tokens, 128] tensors and writes two. Bound by HBM for many
 //     tokens: at 65 536 (26 us for its bytes at the copy rate) the q, k, v
-//     projections take 40 us (52 as three library products), out_proj +
+//     projections take 36 us (52 as three library products), out_proj +
 //     residual + norm 31 (38), the FFN half 41 (66; 49 with erff in its GELU).
 #include "tj_common.h"
 
@@ -340,13 +340,19 @@ __global__ __launch_bounds__(NT, KIND == NARROW_FFN ? 1 : 2) void narrow_kernel(
   }
 }
 
+// Workgroups per weight, n_w weights side by side: never more in all than are
+// resident at once, two of four waves per CU, or one of eight (two weights in
+// LDS). One more (171 x 3 for q, k, v) would start its whole share of the
+// tokens when the others end.
+constexpr int64_t narrow_slots(bool ffn, int n_w) { return (ffn ? 256 : 512) / n_w; }
+static_assert(narrow_slots(true, 1) <= 256 && narrow_slots(false, 1) <= 512 && 2 * narrow_slots(false, 2) <= 512 &&
+              3 * narrow_slots(false, 3) <= 512, "resident workgroups");
+
 template <NarrowKind KIND, Act A>
 int launch_narrow(const NarrowArgs& a, int n_w, hipStream_t stream) {
-  // Resident workgroups: two of four waves per CU, or one of eight (two weights in LDS).
   constexpr int NT = KIND == NARROW_FFN ? 512 : 256;
   const int64_t full = (a.M + NT / 2 - 1) / (NT / 2);  // 32 tokens a wave
-  const int64_t slots = KIND == NARROW_FFN ? 256 : 512;
-  const int64_t per = (slots + n_w - 1) / n_w;
+  const int64_t per = narrow_slots(KIND == NARROW_FFN, n_w);
   hipLaunchKernelGGL((narrow_kernel<KIND, A, NT>), dim3((unsigned)(full < per ? full : per), (unsigned)n_w), dim3(NT), 0,
                      stream, a);
   return tjh::launch_status();

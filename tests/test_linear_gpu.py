@@ -45,6 +45,16 @@ def test_projections(cuda, m, n, k, n_w):
         assert bool(((y.double() - x.double() @ w.double().t()).abs() <= _bound(x, w)).all())
 
 
+@pytest.mark.parametrize("m", [21760, 21761, 21889, 65536])
+def test_three_projections_over_the_whole_chip(cuda, m):
+    """One turn of the resident workgroups (170 per weight, 128 tokens each), and more."""
+    from techjam_amd.kernels.linear import projections
+
+    x, *ws = _draw(cuda, m, (m, 128), *[(128, 128)] * 3)
+    for w, y in zip(ws, projections(x, ws)):
+        assert bool(((y.double() - x.double() @ w.double().t()).abs() <= _bound(x, w)).all())
+
+
 @pytest.mark.parametrize("act", ["gelu", "relu"])
 @pytest.mark.parametrize("m,n,k", [(7, 128, 64), (65, 1024, 256), (40, 32, 512)])
 def test_hidden_layer(cuda, m, n, k, act):
