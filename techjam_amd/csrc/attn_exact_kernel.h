@@ -342,6 +342,9 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
 
   float16_t oacc[QB][TL::DB];
   float m_run[QB], l_run[QB];
+  // A later part may start on keys that all score -inf (k beyond fp16): its
+  // reference stays unset, and is the max of the first tile that has one.
+  [[maybe_unused]] bool unset[QB];
   // -m_run splat kept as a register block: it is the C operand of each query
   // block's first score MFMA, so the scores leave the MFMA already shifted
   // without re-initialising the accumulators every tile.
@@ -350,6 +353,7 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
   for (int qb = 0; qb < QB; ++qb) {
     m_run[qb] = -__builtin_inff();
     l_run[qb] = 0.f;
+    unset[qb] = true;
 #pragma unroll
     for (int r = 0; r < 16; ++r) cneg[qb][r] = 0.f;
 #pragma unroll
@@ -394,6 +398,7 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
       half8_t pf[QB][NS];
       half8_t pl[QB][SPLIT ? NS : 1];  // split heads: p - fp16(p), rounded to fp16
       float shift[QB];
+      bool set[QB];  // this tile sets the row's reference
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
         const int qb0 = qw0 + 32 * qb;
@@ -419,11 +424,15 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
         // Lazy rescaling: the reference point moves only when a row's max grows
         // by more than 2^8 (p <= 256 is exact enough in fp16 and harmless in the
         // fp32 accumulators); the first tile always sets it.
-        shift[qb] = first ? t_max : (t_max > kRescaleLog2 ? t_max : 0.f);
-        // A later part may start on keys that all score -inf (k beyond fp16):
-        // they weigh nothing, as in a sweep that started before them.
         if constexpr (PART) {
-          if (kt0 > 0 && first && t_max == -__builtin_inff()) shift[qb] = 0.f;
+          // While unset, m_run is 0 and nothing has been added up.
+          set[qb] = unset[qb];
+          shift[qb] = set[qb] ? t_max : (t_max > kRescaleLog2 ? t_max : 0.f);
+          unset[qb] = unset[qb] && kt0 > 0 && t_max == -__builtin_inff();
+          if (unset[qb]) shift[qb] = 0.f;
+        } else {
+          set[qb] = first;
+          shift[qb] = first ? t_max : (t_max > kRescaleLog2 ? t_max : 0.f);
         }
       }
       // One wave-wide decision per tile for all query blocks (a lane or block
@@ -434,8 +443,8 @@ __device__ __forceinline__ void attn_tile(const AttnArgs& a, SM& sm, int b, int 
       if (first || __any(moved)) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
-          const float alpha = first ? 0.f : fast_exp2(-shift[qb]);
-          m_run[qb] = first ? shift[qb] : m_run[qb] + shift[qb];
+          const float alpha = set[qb] ? 0.f : fast_exp2(-shift[qb]);
+          m_run[qb] = set[qb] ? shift[qb] : m_run[qb] + shift[qb];
           l_run[qb] *= alpha;
 #pragma unroll
           for (int db = 0; db < TL::DB; ++db)

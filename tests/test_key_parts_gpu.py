@@ -138,3 +138,30 @@ def test_nan_and_infinite_keys_as_in_one_sweep(cuda, causal, dtype):
     assert torch.equal(torch.isnan(got).any(-1), bad)
     tol = 2 * 2 ** -11 * float(v.abs().max()) + (2 ** -10 * float(v.abs().max()) if dtype == torch.float16 else 1e-5)
     assert float((got - want)[~bad].abs().max()) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("level", [-40.0, -200.0, 3.0])
+@pytest.mark.parametrize("dead", [64, 192])
+def test_low_scores_behind_infinite_keys(cuda, dtype, level, dead):
+    """A part that starts on keys scoring -inf weighs its others by their own
+    max: against 2^0, scores around 2^-40 would all round to zero."""
+    from techjam_amd.kernels import _lib, scaled_dot_product_attention
+
+    b, h, s, d = 1, 2, 4096, 64
+    assert _lib.lib().tj_attn_workspace_bytes(b, h, s, d, 1) > 0
+    g = torch.Generator(device=cuda).manual_seed(13)
+    q, k, v = (torch.randn(b, s, h, d, generator=g, device=cuda).to(dtype).transpose(1, 2) for _ in range(3))
+    q[..., 0] = 16.0
+    k[..., 0] = level / 2.885390  # 16 k_0 / 8 log2(e): all scores around 2^level, the same rounding in all
+    for t0 in range(512, s, 512):
+        k[:, :, t0:t0 + dead, 0] = -float("inf")
+    got = scaled_dot_product_attention(q, k, v, is_causal=True)
+    seen = torch.ones(s, s, dtype=torch.bool, device=cuda).tril() & ~torch.isinf(k[0, 0, :, 0])[None]
+    kd = torch.where(torch.isinf(k[0]), 0, k[0]).double()
+    sc = (q[0].double() @ kd.transpose(1, 2).contiguous()) * d ** -0.5
+    ref = torch.softmax(sc.masked_fill(~seen, float("-inf")), -1) @ v[0].double()
+    # P and v rounded to fp16 (2^-11 of max |v| each), scores off by 2^-10 of
+    # the spread of the other dims (below 1.5) and 2^-22 of |level|, fp16 results.
+    tol = float(v.abs().max()) * (2 * 2 ** -11 + 2 * (1.5 * 2 ** -10 + 2 ** -22 * abs(level)) + 2 ** -11)
+    assert float((got[0].double() - ref).abs().max()) <= tol
