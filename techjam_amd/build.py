@@ -43,9 +43,11 @@ FLAGS = [
 ]
 
 
-# Per-file additions. The exact-attention kernel never needs IEEE NaN
-# semantics in its row maxima (scores are finite or -inf), and without them
-# fmaxf chains compile to v_max3 with no canonicalising moves. Its split-score
+# Per-file additions. The exact-attention kernel does without IEEE NaN
+# semantics in its row maxima -- a NaN score reaches its row through the row's
+# sum and products -- and then fmaxf chains compile to v_max3 with no
+# canonicalising moves. What adds its key parts (attn_exact_combine.hip)
+# compares sums that may be NaN and is built with them. Its split-score
 # instance with two query blocks per wave is scheduled by LLVM's max-ILP
 # strategy (faster for it; the default scheduler is faster for the others).
 FILE_FLAGS = {

@@ -82,6 +82,22 @@ struct AttnArgs {
   float* part_ml;  // [B*H*n_parts][128][2]
 };
 
+// Parts of query tile mt, and the tile and part that position j of a (b, h)'s
+// list is. Causal tile mt (128 rows) has 2 (mt + 1) key tiles of 64, so with
+// c = part_tiles / 2 tiles c g .. c g + c - 1 have g + 1 parts.
+__host__ __device__ inline int tile_parts(int mt, int n_keytiles, int part_tiles, int causal) {
+  return causal ? mt / (part_tiles / 2) + 1 : (n_keytiles + part_tiles - 1) / part_tiles;
+}
+__host__ __device__ inline int first_part(int mt, int n_keytiles, int part_tiles, int causal) {
+  if (!causal) return mt * ((n_keytiles + part_tiles - 1) / part_tiles);
+  const int c = part_tiles / 2, g = mt / c;
+  return c * g * (g + 1) / 2 + (mt - c * g) * (g + 1);
+}
+
+// A part's row sum is zero exactly where it has no keys for the row. Tested by
+// bits: NaN sums count as keys, and the part kernels are built without NaN comparisons.
+__device__ __forceinline__ bool has_keys(float sum) { return (__builtin_bit_cast(uint32_t, sum) << 1) != 0; }
+
 // The split-score kernel with two query blocks per wave on 32-key tiles
 // (fp32 inputs, head_dim 64), built in attn_exact_split.hip.
 int launch_split_wide(const AttnArgs& a, hipStream_t stream);
@@ -89,6 +105,10 @@ int launch_split_wide(const AttnArgs& a, hipStream_t stream);
 // The key parts (attn_exact_parts.hip).
 int dispatch_parts_f32(const AttnArgs& a, int64_t D, hipStream_t stream);
 int dispatch_parts_f16(const AttnArgs& a, int64_t D, hipStream_t stream);
+
+// Their sums added up (attn_exact_combine.hip).
+int combine_parts_f32(const AttnArgs& a, int64_t D, hipStream_t stream);
+int combine_parts_f16(const AttnArgs& a, int64_t D, hipStream_t stream);
 
 namespace {
 
@@ -254,10 +274,6 @@ struct KVStage {
     }
   }
 };
-
-// A part's row sum is zero exactly where it has no keys for the row. Tested by
-// bits: NaN sums count as keys, and this file is built without NaN comparisons.
-__device__ __forceinline__ bool has_keys(float sum) { return (__builtin_bit_cast(uint32_t, sum) << 1) != 0; }
 
 // One query tile of one (b, h): 4 waves x 32*QB rows. Each wave holds QB
 // 32-row query blocks, so every K / V^T operand read from LDS feeds QB MFMAs.
@@ -663,24 +679,13 @@ __global__ __launch_bounds__(NT, (HD > 128 ? 1 : 2)) void attn_fwd_kernel(AttnAr
   attn_tile<T, HD, QB, false, BNT>(a, sm, b, h, q0, row_cap, L);
 }
 
-// Parts of query tile mt, and the tile and part that position j of a (b, h)'s
-// list is. Causal tile mt (128 rows) has 2 (mt + 1) key tiles of 64, so with
-// c = part_tiles / 2 tiles c g .. c g + c - 1 have g + 1 parts.
-__host__ __device__ inline int tile_parts(int mt, int n_keytiles, int part_tiles, int causal) {
-  return causal ? mt / (part_tiles / 2) + 1 : (n_keytiles + part_tiles - 1) / part_tiles;
-}
-__host__ __device__ inline int first_part(int mt, int n_keytiles, int part_tiles, int causal) {
-  if (!causal) return mt * ((n_keytiles + part_tiles - 1) / part_tiles);
-  const int c = part_tiles / 2, g = mt / c;
-  return c * g * (g + 1) / 2 + (mt - c * g) * (g + 1);
-}
-
 // Few query tiles: each tile's keys are cut into parts of a.part_tiles key
 // tiles, one workgroup each, so that the launch is as long as a part instead
 // of the longest tile (and covers the chip). Tiles of more than one part leave
 // unnormalised sums, which combine_parts_kernel adds. A part starts at a
 // multiple of 128 keys at or before its tile's first row, so every row sees
-// its first key and the running reference is finite.
+// its first key, and has a reference from its first tile on unless all of that
+// tile's keys score -inf.
 template <typename T, int HD, bool SPLIT_OK>
 __global__ __launch_bounds__(NT, (HD > 128 ? 1 : 2)) void attn_parts_kernel(AttnArgs a) {
   constexpr int BNT = sizeof(T) == 4 && (HD == 256 || (HD == 128 && SPLIT_OK)) ? 32 : 64;
@@ -718,55 +723,6 @@ __global__ __launch_bounds__(NT, (HD > 128 ? 1 : 2)) void attn_parts_kernel(Attn
   attn_tile<T, HD, 1, false, BNT, true>(t, sm, b, h, mt * 128, a.S, L, p * t.part_tiles, slot);
 }
 
-// Adds the parts of one query tile: out = sum_p 2^(m_p - M) O_p / sum_p
-// 2^(m_p - M) l_p (+ v bias), zero for rows at or past the valid length. One
-// row per HD / 4 lanes and thread, the loads of several parts in flight: with
-// a tile's rows and parts one after another its latency was most of the call.
-template <typename T, int HD>
-__global__ __launch_bounds__(NT) void combine_parts_kernel(AttnArgs a) {
-  constexpr int LPR = HD / 4, RPB = NT / LPR;  // lanes per row, rows per workgroup
-  const int tile = blockIdx.x / (128 / RPB);
-  const int bh = tile / a.n_mtiles, mt = tile % a.n_mtiles;
-  const int nk = (a.S + 63) / 64;
-  const int np = tile_parts(mt, nk, a.part_tiles, a.causal);
-  const int r = blockIdx.x % (128 / RPB) * RPB + threadIdx.x / LPR, qi = mt * 128 + r;
-  if (np == 1 || qi >= a.S) return;
-  const int b = bh / a.H, h = bh % a.H;
-  int L = a.S;
-  if (a.valid_len != nullptr) L = min(a.S, max(0, a.valid_len[b]));
-  const int c = 4 * (threadIdx.x % LPR);
-  float4_t y = {0.f, 0.f, 0.f, 0.f};
-  if (qi < L) {
-    using float2_t = float __attribute__((ext_vector_type(2)));
-    const int64_t slot0 = int64_t(bh) * a.n_parts + first_part(mt, nk, a.part_tiles, a.causal);
-    const float2_t* ml = reinterpret_cast<const float2_t*>(a.part_ml) + slot0 * 128 + r;
-    const float* po = a.part_o + (slot0 * 128 + r) * HD + c;
-    float m = -__builtin_inff();
-#pragma unroll 8
-    for (int p = 0; p < np; ++p) {
-      const float2_t x = ml[p * 128];
-      m = has_keys(x[1]) ? fmaxf(m, x[0]) : m;
-    }
-    float l = 0.f;
-#pragma unroll 4
-    for (int p = 0; p < np; ++p) {
-      const float2_t x = ml[p * 128];
-      const float4_t o = *reinterpret_cast<const float4_t*>(po + (int64_t)p * 128 * HD);
-      const float wgt = has_keys(x[1]) ? fast_exp2(x[0] - m) : 0.f;  // a part without keys holds zeros
-      l += wgt * x[1];
-      y += wgt * o;
-    }
-    const float4_t bv = a.v_bias != nullptr ? *reinterpret_cast<const float4_t*>(a.v_bias + h * HD + c) : float4_t{0.f, 0.f, 0.f, 0.f};
-    const bool live = l > 0.f;
-    const float inv = live ? 1.f / l : 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = y[e] * inv + (live ? bv[e] : 0.f);  // NaN stays NaN, as in one sweep
-  }
-  T* op = reinterpret_cast<T*>(a.o) + a.vo.row(b, h, qi) + c;
-  if constexpr (sizeof(T) == 4) *reinterpret_cast<float4_t*>(op) = y;
-  else *reinterpret_cast<half4_t*>(op) = half4_t{(half_t)y[0], (half_t)y[1], (half_t)y[2], (half_t)y[3]};
-}
-
 template <typename T, int HD>
 int launch_parts(AttnArgs a, hipStream_t stream) {
   const int64_t bhn = int64_t(a.B) * a.H, total = bhn * a.n_parts;
@@ -780,9 +736,7 @@ int launch_parts(AttnArgs a, hipStream_t stream) {
   }
   const int rc = tjh::launch_status();
   if (rc != TJ_OK) return rc;
-  hipLaunchKernelGGL((combine_parts_kernel<T, HD>), dim3(uint32_t(bhn * a.n_mtiles * (HD / 8))), dim3(NT), 0,
-                     stream, a);
-  return tjh::launch_status();
+  return sizeof(T) == 4 ? combine_parts_f32(a, HD, stream) : combine_parts_f16(a, HD, stream);
 }
 
 template <typename T, int HD, int QB, int BNT = BN>
