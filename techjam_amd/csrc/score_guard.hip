@@ -45,6 +45,7 @@ struct GuardArgs {
   const void* k;
   View4 vq, vk;
   int H, S, D, n;
+  int first;  // workgroup 0 of this launch
   float scale, ceiling;
   int exact_prefix;
   const int32_t* idx;
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(GP) void score_guard_partial_kernel(GuardArgs a, do
   __shared__ float red_m[GP / kWave];
 
   const int nb = guard_blocks(a.n);
-  const int id = blockIdx.x;
+  const int id = a.first + blockIdx.x;
   const int bh = id / nb, rb = id % nb;
   const int b = bh / a.H, h = bh % a.H;
   const T* qp = reinterpret_cast<const T*>(a.q);
@@ -231,16 +232,23 @@ int guard_launch(const void* q, const void* k, int dtype, int64_t B, int64_t H, 
   a.sigma = sigma_out; a.mean = mean_out; a.smax = smax_out; a.flags = flags_out; a.coeffs = coeffs_out;
   a.row_limit = row_limit_out;
   a.split = split_out;
-  const dim3 grid((unsigned)(B * H * tj::guard_blocks(a.n)));
+  // A launch holds fewer than 2^32 threads: 2^22 workgroups and more (as many
+  // (b, h) at up to 64 samples) run in slices.
+  const int64_t total = B * H * tj::guard_blocks(a.n);
+  constexpr int64_t kSlice = (int64_t(1) << 32) / tj::GP / 2;
   auto partial = [&](auto zero, auto nc) {
-    hipLaunchKernelGGL((tj::score_guard_partial_kernel<decltype(zero), decltype(nc)::value>), grid, dim3(tj::GP), 0,
-                       stream, a, partials);
+    for (int64_t first = 0; first < total; first += kSlice) {
+      a.first = (int)first;
+      hipLaunchKernelGGL((tj::score_guard_partial_kernel<decltype(zero), decltype(nc)::value>),
+                         dim3((unsigned)(total - first < kSlice ? total - first : kSlice)), dim3(tj::GP), 0, stream, a, partials);
+      if (const int rc = tjh::launch_status(); rc != TJ_OK) return rc;
+    }
+    return (int)TJ_OK;
   };
   constexpr std::integral_constant<int, 8> narrow;
   constexpr std::integral_constant<int, tj::GMAXD / 8> wide;
-  if (dtype == TJ_F32) D <= 64 ? partial(float(), narrow) : partial(float(), wide);
-  else D <= 64 ? partial(half_t(), narrow) : partial(half_t(), wide);
-  const int rc = tjh::launch_status();
+  const int rc = dtype == TJ_F32 ? (D <= 64 ? partial(float(), narrow) : partial(float(), wide))
+                                 : (D <= 64 ? partial(half_t(), narrow) : partial(half_t(), wide));
   if (rc != TJ_OK) return rc;
   const int bhn = (int)(B * H);
   hipLaunchKernelGGL(tj::score_guard_final_kernel, dim3((unsigned)((bhn + tj::GT - 1) / tj::GT)), dim3(tj::GT), 0,

@@ -38,3 +38,21 @@ def test_moments_match_the_oracle(cuda, b, h, n, d, dtype):
         assert torch.allclose(res.sigma.cpu().double(), ref, rtol=1e-4, atol=1e-6)
     else:
         assert res.flags.cpu().tolist() == [0] * (b * h)  # one score has no spread
+
+
+def test_more_heads_than_one_launch_holds(cuda):
+    """2^22 workgroups of 1024 threads exceed a launch: the sums run in slices."""
+    from techjam_amd.kernels import score_guard
+
+    h, n, d = (1 << 22) + 5, 2, 4
+    g = torch.Generator(device=cuda).manual_seed(1)
+    q, k = (torch.randn(1, h, n, d, generator=g, device=cuda, dtype=torch.float16) for _ in range(2))
+    res = score_guard(q, k, 0.5, ceiling=0.4)
+    torch.cuda.synchronize()
+    s = (q[0].float() @ k[0].float().transpose(-2, -1).contiguous()).double() * 0.5  # exact products, four-term sums
+    assert torch.allclose(res.mean.double(), s.mean(dim=(-1, -2)), rtol=0, atol=1e-6)
+    sd = s.flatten(1).std(dim=1)
+    # fp32 squares of scores up to 20, cancelling against the mean's
+    assert float((res.sigma.double() - sd).abs().max()) <= 2e-3
+    clear = (sd - 0.4).abs() > 2e-3
+    assert torch.equal((res.flags == 1)[clear], (sd <= 0.4)[clear])
