@@ -23,7 +23,8 @@ HIP kernels actually holds per batch item at its peak:
   activations (before and after GELU), so the larger of the two is counted.
 
 The caller's output buffer for the whole batch is reserved first, as in the
-reference, and a fixed allowance covers the GEMM libraries' workspaces. The
+reference, and a fixed allowance covers the GEMM libraries' workspaces and the
+exact kernel's sums of key parts (at most 47 MiB, for few heads). The
 chunk is the largest power of two whose items fit what is left -- powers of
 two keep the out-of-memory halving of ``forward_batch_chunks`` on the same
 sizes.
@@ -40,8 +41,9 @@ from ..kernels import _lib
 
 DEFAULT_MEMORY_FRACTION = 0.85
 #: Allowance for workspaces the GEMM libraries take from torch's allocator
-#: on first use (hipBLASLt / rocBLAS) and for the small per-call tensors
-#: (valid lengths, the guard's cached row sample).
+#: on first use (hipBLASLt / rocBLAS), for the sums of key parts
+#: (``tj_attn_workspace_bytes``) and for the small per-call tensors (valid
+#: lengths, the guard's cached row sample).
 LIBRARY_ALLOWANCE_BYTES = 256 << 20
 GUARD_OUTPUT_BYTES_PER_HEAD = 4 * (1 + 1 + 1 + 1 + 3 + 1 + 1)  # sigma, mean, smax, flag, 3 coeffs, limit, split
 GUARD_SAMPLES = 512
@@ -96,12 +98,16 @@ def attention_core_bytes(batch: int, num_heads: int, seq_len: int, head_dim: int
                          element_size: int = 4) -> int:
     """Bytes ``guarded_attention`` (``poly``) or the exact kernel allocates for
     resident q, k, v: the output, plus on the guarded route the polynomial
-    workspace and the guard's workspace and outputs."""
+    workspace and the guard's workspace and outputs, and on the exact one the
+    sums of key parts (few query tiles with long sweeps, causal or not)."""
     heads = batch * num_heads
     total = heads * seq_len * head_dim * element_size
     if poly:
         total += heads * (poly_workspace_bytes_per_head() + guard_workspace_bytes_per_head()
                           + GUARD_OUTPUT_BYTES_PER_HEAD)
+    else:
+        total += max(int(_lib.lib().tj_attn_workspace_bytes(batch, num_heads, seq_len, head_dim, causal))
+                     for causal in (0, 1))
     return total
 
 
