@@ -48,6 +48,11 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+#: Sequences up to which the library never cuts a sweep into parts (the
+#: shortest part and what a sweep must be longer by, 20 key tiles of 64 in
+#: all), so that short calls do not ask for the workspace's size.
+ONE_SWEEP_MAX_SEQ = 1216
+
 #: The kernels address the rows of one (b, h) with 31-bit byte offsets.
 MAX_HEAD_SPAN_BYTES = 1 << 31
 
@@ -189,8 +194,8 @@ def scaled_dot_product_attention(
     if row_limit is None:
         # Long sweeps over few query tiles are cut into parts, whose sums need
         # a workspace; 0 bytes for all other calls.
-        # (never below 20 key tiles of 64, so short calls do not ask).
-        ws_bytes = _lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(bool(is_causal))) if s > 1216 else 0
+        ws_bytes = (_lib.lib().tj_attn_workspace_bytes(b, h, s, d, int(bool(is_causal)))
+                    if s > ONE_SWEEP_MAX_SEQ else 0)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
         code = _lib.lib().tj_attn_fwd_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],

@@ -26,3 +26,12 @@ def test_the_sums_fit_the_allowance(d):
     sizes = [*range(1216, 60000, 320), *range(60000, 600000, 8192)]
     most = max(_bytes(1, h, s, d, c) for h in (1, 2, 3, 5, 8, 13, 32, 64, 128) for s in sizes for c in (0, 1))
     assert 0 < most <= 47 << 20 < planner.LIBRARY_ALLOWANCE_BYTES // 4
+
+
+def test_short_calls_need_not_ask():
+    """The largest sequence that no shape cuts into parts, exactly."""
+    from techjam_amd.kernels.attention import ONE_SWEEP_MAX_SEQ, SUPPORTED_HEAD_DIMS
+
+    shapes = [(h, d, c) for h in (1, 2, 4, 8, 16, 64) for d in SUPPORTED_HEAD_DIMS for c in (0, 1)]
+    assert not any(_bytes(1, h, s, d, c) for h, d, c in shapes for s in range(1, ONE_SWEEP_MAX_SEQ + 1))
+    assert any(_bytes(1, h, ONE_SWEEP_MAX_SEQ + 1, d, c) for h, d, c in shapes)
