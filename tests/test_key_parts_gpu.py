@@ -33,7 +33,7 @@ def _one_sweep(q, k, v, causal, lengths, q_bias, v_bias):
     (1, 1, 1281, 64, torch.float32), (1, 2, 2048, 64, torch.float16), (2, 3, 2049, 64, torch.float32),
     (1, 1, 5000, 32, torch.float16), (1, 4, 3583, 128, torch.float32), (1, 1, 2177, 128, torch.float16),
     (1, 2, 2500, 256, torch.float32), (1, 9, 4096, 64, torch.float16), (1, 1, 1537, 256, torch.float16), (1, 1, 2176, 64, torch.float32),
-    (1, 1, 16384, 64, torch.float32)])
+    (1, 1, 16384, 64, torch.float32), (2, 2, 2049, 64, torch.float32)])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("padded,biased", [(False, False), (True, True)])
 def test_parts_add_up(cuda, b, h, s, d, dtype, causal, padded, biased):

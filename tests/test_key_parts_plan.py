@@ -35,3 +35,14 @@ def test_short_calls_need_not_ask():
     shapes = [(h, d, c) for h in (1, 2, 4, 8, 16, 64) for d in SUPPORTED_HEAD_DIMS for c in (0, 1)]
     assert not any(_bytes(1, h, s, d, c) for h, d, c in shapes for s in range(1, ONE_SWEEP_MAX_SEQ + 1))
     assert any(_bytes(1, h, ONE_SWEEP_MAX_SEQ + 1, d, c) for h, d, c in shapes)
+
+
+@pytest.mark.parametrize("h,s,d,causal,parts", [
+    (1, 2048, 64, 1, True), (1, 16384, 64, 1, True), (8, 2048, 64, 1, True), (4, 4096, 128, 1, True), (4, 1257, 64, 1, True),
+    # 2.5 parts' length and more, but the sums of that many parts cost what they save
+    (16, 1375, 64, 0, False), (8, 2863, 64, 0, False), (12, 2014, 128, 0, False), (108, 1256, 32, 1, False),
+    # less than 2.5
+    (16, 4096, 64, 1, False), (32, 2048, 64, 1, False),
+])
+def test_where_parts_pay(h, s, d, causal, parts):
+    assert (_bytes(1, h, s, d, causal) > 0) == parts
