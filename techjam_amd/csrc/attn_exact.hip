@@ -46,15 +46,17 @@ int launch(const AttnArgs& a, hipStream_t stream) {
 
 // Key parts, where the longest key sweep of a 128-row query tile is at least
 // 2.5 times what an even split of all key tiles over the chip's workgroup
-// slots gives, and longer than a part by two key tiles and one for every 18
-// parts whose sums go through memory; part_tiles 0: none. Measured (us, one
+// slots gives, and (below head_dim 256) longer than a part by two key tiles and
+// one for every 18 parts whose sums go through memory; part_tiles 0: none. Measured (us, one
 // sweep -> parts, causal, head_dim 64 fp32): 1 head of 2048 33 -> 16, of 8192
 // 114 -> 31, of 16 384 224 -> 74; 4 heads of 4096 61 -> 31, 8 of 2048 34 -> 25.
 // Past the first line the parts cost as much as they save: 16 heads of 4096
 // fp32 73 -> 73, fp16 68 -> 69, head_dim 128 121 -> 132 and 105 -> 121; 32 of
-// 2048 40 -> 46, fp16 36 -> 43. The second is that of 650 random calls near it
-// (all head dims and types, padded and not): without it 56 were slower in
-// parts, 16 heads of 1375 not causal 26 -> 32, 12 of 2014 x 128 62 -> 66.
+// 2048 40 -> 46, fp16 36 -> 43. The second is that of 1400 random calls near it
+// (all head dims and types, half of them padded): without it 137 were slower in
+// parts, 16 heads of 1375 not causal 26 -> 32, 12 of 2014 x 128 62 -> 66; with
+// it 11, all padded to about twice their length, and none at head_dim 256
+// either way.
 struct PartPlan {
   int part_tiles = 0, n_parts = 0, n_mtiles = 0;
 };
@@ -72,7 +74,7 @@ PartPlan plan_parts(int64_t B, int64_t H, int64_t S, int64_t D, int causal) {
   if (nk < part + kPartGain || 2 * nk < 5 * part) return p;
   const int64_t n_parts = first_part((int)nm, (int)nk, (int)part, causal);
   const int64_t whole = causal ? (nm < part / 2 ? nm : part / 2) : 0;  // tiles of one part
-  if (18 * (nk - part - 2) < bhn * (n_parts - whole)) return p;
+  if (D != 256 && 18 * (nk - part - 2) < bhn * (n_parts - whole)) return p;
   p.part_tiles = (int)part;
   p.n_mtiles = (int)nm;
   p.n_parts = (int)n_parts;

@@ -41,6 +41,7 @@ def test_short_calls_need_not_ask():
     (1, 2048, 64, 1, True), (1, 16384, 64, 1, True), (8, 2048, 64, 1, True), (4, 4096, 128, 1, True), (4, 1257, 64, 1, True),
     # 2.5 parts' length and more, but the sums of that many parts cost what they save
     (16, 1375, 64, 0, False), (8, 2863, 64, 0, False), (12, 2014, 128, 0, False), (108, 1256, 32, 1, False),
+    (6, 1600, 256, 0, True),  # not at head_dim 256
     # less than 2.5
     (16, 4096, 64, 1, False), (32, 2048, 64, 1, False),
 ])
