@@ -18,9 +18,8 @@ __global__ __launch_bounds__(NT) void combine_parts_kernel(AttnArgs a) {
   const int tile = blockIdx.x / (128 / RPB);
   const int bh = tile / a.n_mtiles, mt = tile % a.n_mtiles;
   const int nk = (a.S + 63) / 64;
-  const int np = tile_parts(mt, nk, a.part_tiles, a.causal);
   const int r = blockIdx.x % (128 / RPB) * RPB + threadIdx.x / LPR, qi = mt * 128 + r;
-  if (np == 1 || qi >= a.S) return;
+  if (tile_parts(mt, nk, a.part_tiles, a.causal) == 1 || qi >= a.S) return;
   const int b = bh / a.H, h = bh % a.H;
   int L = a.S;
   if (a.valid_len != nullptr) L = min(a.S, max(0, a.valid_len[b]));
@@ -31,6 +30,7 @@ __global__ __launch_bounds__(NT) void combine_parts_kernel(AttnArgs a) {
     const int64_t slot0 = int64_t(bh) * a.n_parts + first_part(mt, nk, a.part_tiles, a.causal);
     const float2_t* ml = reinterpret_cast<const float2_t*>(a.part_ml) + slot0 * 128 + r;
     const float* po = a.part_o + (slot0 * 128 + r) * HD + c;
+    const int np = live_parts(mt, L, a.part_tiles, a.causal);
     float m = -__builtin_inff();
 #pragma unroll 8
     for (int p = 0; p < np; ++p) {
