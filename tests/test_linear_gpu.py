@@ -135,3 +135,86 @@ def test_autocast_decides_the_type_of_the_attention_context(cuda):
     with torch.autocast("cuda", torch.float16):
         assert attn.context(x).dtype == torch.float16
     assert attn.context(x).dtype == torch.float32
+
+
+def test_width_128_ffn_with_relu(cuda):
+    from techjam_amd.kernels.linear import ffn_norm
+
+    b, s = 2, 12301
+    x, r, w, w2, bi, bo, *g = _draw(cuda, 5, (b, s, 128), (b, s, 128), (128, 128), (128, 128), (128,), (128,), (128,),
+                                    (128,))
+    norm, xs = _norm(cuda, g), x.reshape(-1, 128)
+    h = F.relu(xs.double() @ w.double().t() + bi.double())
+    hidden = _bound(xs, w) + 1e-6 * (1 + h)
+    bound = (hidden @ w2.double().abs().t() + _bound(h + hidden, w2)).view(b, s, 128)
+    ref = r.double() + (h @ w2.double().t() + bo.double()).view(b, s, 128)
+    _check_residual(ffn_norm(x, w, bi, "relu", w2, bo, r, None, 0, norm), ref, bound, norm)
+
+
+@pytest.mark.parametrize("tokens", [1, 31, 4100])
+def test_sum_in_place_or_not_stored(cuda, tokens):
+    """The two forms of ``out`` that only the C entry points offer: the
+    residual itself, and none."""
+    from techjam_amd.kernels import _lib
+    from techjam_amd.kernels.attention import _stream_ptr
+
+    x, r, w, w2, bi, bo, ga, be = _draw(cuda, tokens, (tokens, 128), (tokens, 128), (128, 128), (128, 128), (128,),
+                                        (128,), (128,), (128,))
+    lib, stream = _lib.lib(), _stream_ptr(x.device)
+
+    def residual(resid, out, ln):
+        return lib.tj_narrow_residual_norm(x.data_ptr(), w.data_ptr(), bo.data_ptr(), resid.data_ptr(), out, tokens, tokens,
+                                           None, 0, ga.data_ptr(), be.data_ptr(), ln.data_ptr(), 1e-5, 0, stream)
+
+    def ffn(resid, out, ln):
+        return lib.tj_narrow_ffn_norm(x.data_ptr(), w.data_ptr(), bi.data_ptr(), 2, w2.data_ptr(), bo.data_ptr(),
+                                      resid.data_ptr(), out, tokens, tokens, None, 0, ga.data_ptr(), be.data_ptr(),
+                                      ln.data_ptr(), 1e-5, 0, stream)
+
+    for call in (residual, ffn):
+        out, ln = torch.empty_like(r), torch.empty_like(r)
+        assert call(r, out.data_ptr(), ln) == 0
+        inplace, ln_in = r.clone(), torch.empty_like(r)
+        assert call(inplace, inplace.data_ptr(), ln_in) == 0
+        ln_only = torch.empty_like(r)
+        assert call(r, None, ln_only) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(inplace, out) and torch.equal(ln_in, ln) and torch.equal(ln_only, ln)
+        assert bool(torch.isfinite(ln).all())
+
+
+@pytest.mark.parametrize("m,n,k,n_w", [(256, 256, 256, 1), (96, 128, 512, 3), (30000, 128, 128, 1), (30000, 128, 128, 3)])
+def test_infinities_nan_and_huge_values(cuda, m, n, k, n_w):
+    """An infinite or NaN input, or one past bf16's largest, makes its row NaN
+    (the low part of an infinity is inf - inf), as in the library's fast mode;
+    the other rows do not see it."""
+    from techjam_amd.kernels.linear import projections
+
+    x, *ws = _draw(cuda, n + k, (m, k), *[(n, k)] * n_w)
+    rows = [3, 7, 11, 20, m - 1]
+    for row, value in zip(rows, (float("inf"), float("nan"), 3.4e38, -float("inf"), -3.4e38)):
+        x[row, row % k] = value
+    clean = torch.ones(m, dtype=torch.bool, device=cuda)
+    clean[rows] = False
+    for w, y in zip(ws, projections(x, ws)):
+        assert bool(torch.isnan(y[rows]).all())
+        assert bool(torch.equal(torch.isnan(y), torch.isnan(F.linear(x, w))))
+        assert bool(((y[clean].double() - x[clean].double() @ w.double().t()).abs() <= _bound(x[clean], w)).all())
+
+
+def test_a_nan_token_stays_in_its_row_of_a_width_128_block(cuda):
+    from techjam_amd.kernels.linear import ffn_norm, residual_norm
+
+    b, s = 1, 24576
+    x, r, w, w2, bi, bo, *g = _draw(cuda, 9, (b, s, 128), (b, s, 128), (128, 128), (128, 128), (128,), (128,), (128,),
+                                    (128,))
+    norm = _norm(cuda, g)
+    lengths = torch.tensor([s - 10], dtype=torch.int32, device=cuda)
+    clean = [t.clone() for t in (*residual_norm(x, w, bo, r, lengths, 2, norm),
+                                 *ffn_norm(x, w, bi, "gelu", w2, bo, r, lengths, 2, norm))]
+    x[0, 100, 5], x[0, s - 1, 7] = float("nan"), float("inf")  # a valid row and a padded one
+    got = (*residual_norm(x, w, bo, r, lengths, 2, norm), *ffn_norm(x, w, bi, "gelu", w2, bo, r, lengths, 2, norm))
+    for was, now in zip(clean, got):
+        assert bool(torch.isnan(now[0, 100]).all())
+        now[0, 100] = was[0, 100]
+        assert torch.equal(now, was)  # the padded row is zeroed, not multiplied by zero
