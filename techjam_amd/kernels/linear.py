@@ -20,23 +20,17 @@ from .attention import _stream_ptr
 #: Width of the layers the one-pass kernels take.
 NARROW = 128
 #: Multiply-adds up to which the small-tile kernel is used, and its depth (at
-#: K = 1024 and 256 x 256 the library takes 9.5 us, this 10.2). One product, us
-#: by the library / here, replayed as graphs: 32 x 256 x 256 11.0 / 4.4, 256 x
-#: 256 x 256 26.0 / 4.5, 256 x 512 x 512 7.5 / 6.4, 1200 x 128 x 512 7.5 / 6.5;
-#: past the line 1200 x 512 x 512 11.2 / 17.2.
+#: K = 1024 and 256 x 256 the library takes 9.5 us, this 10.2). One product, us by the library / here, replayed as graphs: 32 x 256 x
+#: 256 11.0 / 4.4, 256 x 256 x 256 26.0 / 4.5, 256 x 512 x 512 7.5 / 6.4, 1200
+#: x 128 x 512 7.5 / 6.5; past the line 1200 x 512 x 512 11.2 / 17.2.
 ROWS_MAX_WORK = 1 << 26
 ROWS_MAX_K = 512
 #: Tokens from which the one-pass kernels beat a product and the passes after
 #: it, and up to which the shorter one does (us, library + passes / here:
-#: residual + norm 16 384 tokens 17.2 / 17.5, 24 576 21.7 / 19.0, 98 304 57 / 44,
-#: 131 072 72 / 74, 262 144 150 / 162; FFN 30.7 / 30.7, 34 / 32, 95 / 61, 125 /
-#: 78, 259 / 166): below, one tile's latency is all there is; above, the
-#: tensors outgrow the memory-side cache, and the sum in a buffer of its own
-#: costs what the pass saves.
+#: residual + norm 16 384 tokens 16.4 / 16.4, 65 536 38 / 31, 262 144 146 / 155;
+#: FFN 30 / 38, 66 / 41, 249 / 205): below, one tile's latency is all there is.
 NARROW_MIN_TOKENS = 24576
-NARROW_RESIDUAL_MAX_TOKENS = 98304
-#: Tokens from which a lone product of width 128 does.
-NARROW_LONE_MIN_TOKENS = 28672
+NARROW_RESIDUAL_MAX_TOKENS = 131072
 
 
 #: The setting float32 GEMMs on the GPU obey (``torch.backends.cuda.matmul.
@@ -73,42 +67,20 @@ def _usable(x: torch.Tensor, *params: torch.Tensor) -> bool:
     return True
 
 
-def _kernel_for(m: int, n: int, k: int, n_w: int, act: bool) -> Optional[int]:
-    """0 for the small-tile kernel, 1 for the width-128 one, ``None`` where the
-    library is as fast or the shape fits neither. Both are ahead by one or two
-    launches for several weights and with an activation; a lone product (us,
-    library / here) stays with the library
-
-    * at K = 64 from 2^25 on (twice the stores for the work: 4096 x 128 4.8 /
-      4.0, 8192 x 128 5.1 / 5.9, 2048 x 512 4.8 / 5.9),
-    * of up to 16 rows by 512 columns and more at K >= 256, where it reads the
-      weight once without tiles (16 x 512 x 512 4.7 / 5.8, 4 x 1024 x 256 3.9 /
-      4.1; 32 x 512 x 512 7.5 / 6.5, 16 x 256 x 256 8.6 / 4.4),
-    * at width 128 between the two kernels' ranges (4098 rows 5.8 / 7.6, 16 384
-      8.0 / 8.8, 24 576 9.4 / 9.6, 28 672 10.5 / 9.9, 131 073 32.7 / 25.8).
-    """
-    lone = n_w == 1 and not act
-    work = m * n * k * n_w
-    if work <= ROWS_MAX_WORK:
-        if n & 31 or k & 63 or k > ROWS_MAX_K:
-            return None
-        if lone and ((k == 64 and work > ROWS_MAX_WORK // 2) or (m <= 16 and n >= 512 and k >= 256)):
-            return None
-        return 0
-    if n == NARROW and k == NARROW and not act and (not lone or m >= NARROW_LONE_MIN_TOKENS):
-        return 1
-    return None
-
-
 def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional[torch.Tensor] = None,
                 act: Optional[str] = None) -> Optional[Tuple[torch.Tensor, ...]]:
     """``x @ w.T`` for up to three weights of one shape in one launch, or
     ``act(x @ w.T + bias)`` for one (``act`` "gelu" or "relu")."""
     n, k = weights[0].shape
-    m = x.numel() // k if k else 0
-    narrow = _kernel_for(m, n, k, len(weights), act is not None)
-    if narrow is None:
+    if x.numel() * n * len(weights) <= ROWS_MAX_WORK:
+        if n & 31 or k & 63 or k > ROWS_MAX_K:
+            return None
+        narrow = 0
+    elif n == NARROW and k == NARROW and act is None:
+        narrow = 1
+    else:
         return None
+    m = x.numel() // k
     if (x.shape[-1] != k or m == 0 or not _usable(x, *weights, *(() if bias is None else (bias,)))
             or any(w.shape != (n, k) for w in weights) or (bias is not None and bias.shape != (n,))):
         return None  # the kernel reads n values of the bias

@@ -53,23 +53,3 @@ def test_a_bias_of_another_size_stays_off_the_kernel(monkeypatch, size):
     monkeypatch.setattr(linear._lib, "lib", lambda: pytest.fail("the kernel would be called"))
     x, w = torch.zeros(4, 128), torch.zeros(64, 128)
     assert linear.projections(x, (w,), torch.zeros(size), "gelu") is None
-
-
-@pytest.mark.parametrize("m,n,k,n_w,act,kernel", [
-    # one product: where the small-tile kernel measured behind the library
-    (4096, 128, 64, 1, False, 0), (4097, 128, 64, 1, False, None), (8192, 128, 64, 1, False, None),
-    (8192, 128, 64, 1, True, 0), (2730, 128, 64, 3, False, 0),
-    (16, 512, 512, 1, False, None), (17, 512, 512, 1, False, 0), (16, 512, 512, 3, False, 0), (16, 512, 512, 1, True, 0),
-    (16, 256, 512, 1, False, 0), (1, 1024, 256, 1, False, None), (1, 1024, 128, 1, False, 0),
-    # width 128, between the two kernels
-    (4096, 128, 128, 1, False, 0), (4097, 128, 128, 1, False, None), (28671, 128, 128, 1, False, None),
-    (28672, 128, 128, 1, False, 1), (1 << 20, 128, 128, 1, False, 1), (4097, 128, 128, 2, False, 1),
-    (4097, 128, 128, 1, True, None),
-    # neither kernel's shapes
-    (64, 48, 64, 1, False, None), (64, 64, 96, 1, False, None), (4, 64, 1024, 1, False, None),
-    (1 << 20, 256, 256, 3, False, None),
-])
-def test_which_kernel_a_product_takes(m, n, k, n_w, act, kernel):
-    from techjam_amd.kernels.linear import _kernel_for
-
-    assert _kernel_for(m, n, k, n_w, act) == kernel
