@@ -3,9 +3,10 @@
 They do the arithmetic of hipBLASLt's fast float32 mode (operands split into
 two bf16 parts, three products, fp32 accumulation; same error against 64
 bits), so they are used only where a float32 product would run in that mode
-(:func:`fast_float32_matmul`) and, as a raw kernel call records no graph, only
-while gradients are off. Each function returns ``None`` for what it does not
-take or is not faster at, and the caller then uses the library.
+and, as a raw kernel call records no graph, only while gradients are off
+(:func:`split_products_allowed`, which a caller of several of them asks once
+and hands on as ``allowed``). Each function returns ``None`` for what it does
+not take or is not faster at, and the caller then uses the library.
 """
 
 from __future__ import annotations
@@ -33,46 +34,53 @@ NARROW_MIN_TOKENS = 24576
 NARROW_RESIDUAL_MAX_TOKENS = 131072
 
 
-#: The setting float32 GEMMs on the GPU obey (``torch.backends.cuda.matmul.
-#: fp32_precision``, at a third of that property's cost); ``None`` on a torch
-#: without it.
-_fp32_precision = getattr(torch._C, "_get_fp32_precision_getter", None)
+_ACT = {None: 0, "gelu": 1, "relu": 2}
+_NONE = (None, None, None)
+_HIPBLASLT = torch._C._BlasBackend.Cublaslt.value
 
 
-def fast_float32_matmul() -> bool:
-    """Whether a float32 product on the GPU runs on split bf16 operands.
+def split_products_allowed() -> bool:
+    """Whether a float32 ``F.linear`` on the GPU would run here and now on
+    split bf16 operands, with a float32 result and no graph to record.
 
-    That is hipBLASLt's fast mode: the other BLAS backends compute in plain
-    float32 at any setting (256 x 256 x 256: 2.9e-7 of error, split 4.4e-6).
-    ``torch.get_float32_matmul_precision()`` does not tell -- it still says
-    "high" after ``torch.backends.cuda.matmul.fp32_precision`` was set to
-    "ieee", and raises where the two disagree the other way.
+    The split form is hipBLASLt's fast mode: the other BLAS backends compute in
+    plain float32 at any setting (256 x 256 x 256: 2.9e-7 of error, split
+    4.4e-6). ``torch.get_float32_matmul_precision()`` does not tell the mode --
+    it still says "high" after ``torch.backends.cuda.matmul.fp32_precision`` was
+    set to "ieee", and raises where the two disagree the other way.
     """
-    if _fp32_precision is None:
-        fast = torch.get_float32_matmul_precision() != "highest"
-    else:
-        fast = _fp32_precision("cuda", "matmul") == "tf32"
-    return fast and torch._C._get_blas_preferred_backend() == torch._C._BlasBackend.Cublaslt
-
-
-def _usable(x: torch.Tensor, *params: torch.Tensor) -> bool:
-    if (not x.is_cuda or x.dtype != torch.float32 or torch.is_grad_enabled()
-            or not fast_float32_matmul() or not x.is_contiguous() or x.data_ptr() % 16
-            or torch.is_autocast_enabled("cuda")):  # the product would give the autocast type
+    if torch.is_grad_enabled() or torch.is_autocast_enabled():  # autocast: the result has its type
         return False
-    dev = x.device
-    for p in params:
-        if (p is None or p.dtype != torch.float32 or p.device != dev or not p.is_contiguous() or p.data_ptr() % 16):
-            return False
-    return True
+    try:
+        fast = torch._C._get_cublas_allow_tf32()  # a quarter of the cost of fp32_precision
+    except RuntimeError:  # the older and the newer setting disagree; the GEMMs obey the newer
+        fast = torch.backends.cuda.matmul.fp32_precision == "tf32"
+    return fast and torch._C._get_blas_preferred_backend().value == _HIPBLASLT
+
+
+def _usable(allowed: Optional[bool], x: torch.Tensor, *params: torch.Tensor) -> Optional[list]:
+    """The addresses of ``x`` and ``params`` if the kernels may run on them."""
+    if not x.is_cuda or not (split_products_allowed() if allowed is None else allowed):
+        return None
+    dev, f32, ptrs = x.get_device(), torch.float32, []
+    for t in (x, *params):
+        if t is None or t.dtype != f32 or t.get_device() != dev or not t.is_contiguous():
+            return None
+        p = t.data_ptr()
+        if p & 15:
+            return None
+        ptrs.append(p)
+    return ptrs
 
 
 def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional[torch.Tensor] = None,
-                act: Optional[str] = None) -> Optional[Tuple[torch.Tensor, ...]]:
+                act: Optional[str] = None, allowed: Optional[bool] = None) -> Optional[Tuple[torch.Tensor, ...]]:
     """``x @ w.T`` for up to three weights of one shape in one launch, or
     ``act(x @ w.T + bias)`` for one (``act`` "gelu" or "relu")."""
-    n, k = weights[0].shape
-    if x.numel() * n * len(weights) <= ROWS_MAX_WORK:
+    # Plain statements: small blocks are bound by this function's own cost.
+    w_shape, n_w, size = weights[0].shape, len(weights), x.numel()
+    n, k = w_shape
+    if size * n * n_w <= ROWS_MAX_WORK:
         if n & 31 or k & 63 or k > ROWS_MAX_K:
             return None
         narrow = 0
@@ -80,37 +88,48 @@ def projections(x: torch.Tensor, weights: Sequence[torch.Tensor], bias: Optional
         narrow = 1
     else:
         return None
-    m = x.numel() // k
-    if (x.shape[-1] != k or m == 0 or not _usable(x, *weights, *(() if bias is None else (bias,)))
-            or any(w.shape != (n, k) for w in weights) or (bias is not None and bias.shape != (n,))):
-        return None  # the kernel reads n values of the bias
-    outs = [torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device) for _ in weights]
-    ptrs = [w.data_ptr() for w in weights] + [None] * (3 - len(weights))
-    optr = [o.data_ptr() for o in outs] + [None] * (3 - len(weights))
-    code = _lib.lib().tj_linear(x.data_ptr(), *ptrs, *optr, m, n, k, None if bias is None else bias.data_ptr(),
-                                {None: 0, "gelu": 1, "relu": 2}[act], narrow, _stream_ptr(x.device))
-    _lib.check(code, "tj_linear")
+    shape = x.shape
+    if shape[-1] != k or size == 0:
+        return None
+    for w in weights:
+        if w.shape != w_shape:
+            return None
+    if bias is None:
+        ptrs = _usable(allowed, x, *weights)
+    elif bias.shape == (n,):  # the kernel reads n values
+        ptrs = _usable(allowed, x, *weights, bias)
+    else:
+        return None
+    if ptrs is None:
+        return None
+    out_shape = (*shape[:-1], n)
+    outs = [x.new_empty(out_shape) for _ in weights]
+    pad = _NONE[n_w:]
+    code = _lib.lib().tj_linear(*ptrs[:1 + n_w], *pad, *[o.data_ptr() for o in outs], *pad, size // k, n, k,
+                                None if bias is None else ptrs[-1], _ACT[act], narrow, _stream_ptr(x.device))
+    if code:
+        _lib.check(code, "tj_linear")
     return tuple(outs)
 
 
-def _residual_ok(x, resid, bias, valid_len, norm, params) -> bool:
+def _residual_ok(allowed, x, resid, weights, biases, valid_len, norm) -> bool:
     return (x.ndim == 3 and x.shape[-1] == NARROW and x.numel() > 0 and resid.shape == x.shape
-            and all(p is not None and p.shape == (NARROW, NARROW) for p in params)
-            and bias is not None and bias.shape == (NARROW,)
+            and all(w is not None and w.shape == (NARROW, NARROW) for w in weights)
+            and all(b is not None and b.shape == (NARROW,) for b in biases)
             and isinstance(norm, torch.nn.LayerNorm) and tuple(norm.normalized_shape) == (NARROW,)
             and norm.weight is not None and norm.bias is not None
-            and _usable(x, resid, bias, norm.weight, norm.bias, *params)
+            and _usable(allowed, x, resid, norm.weight, norm.bias, *weights, *biases) is not None
             and (valid_len is None or (valid_len.dtype == torch.int32 and valid_len.shape == (x.shape[0],)
                                        and valid_len.device == x.device and valid_len.is_contiguous())))
 
 
 def residual_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, resid: torch.Tensor,
                   valid_len: Optional[torch.Tensor], mode: int, norm: torch.nn.LayerNorm,
-                  zero_padded_norm: bool = False):
+                  zero_padded_norm: bool = False, allowed: Optional[bool] = None):
     """``kernels.elementwise.bias_residual_layernorm`` of ``y = x @ weight.T``
     in one pass, for layers of width 128: ``(out, norm(out))``."""
     if (not NARROW_MIN_TOKENS <= x.numel() // NARROW <= NARROW_RESIDUAL_MAX_TOKENS
-            or not _residual_ok(x, resid, bias, valid_len, norm, (weight,))):
+            or not _residual_ok(allowed, x, resid, (weight,), (bias,), valid_len, norm)):
         return None
     out, ln = torch.empty_like(resid), torch.empty_like(resid)
     code = _lib.lib().tj_narrow_residual_norm(
@@ -123,16 +142,15 @@ def residual_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, res
 
 def ffn_norm(x: torch.Tensor, w_in: torch.Tensor, b_in: torch.Tensor, act: str, w_out: torch.Tensor,
              bias: torch.Tensor, resid: torch.Tensor, valid_len: Optional[torch.Tensor], mode: int,
-             norm: torch.nn.LayerNorm, zero_padded_norm: bool = False):
+             norm: torch.nn.LayerNorm, zero_padded_norm: bool = False, allowed: Optional[bool] = None):
     """The same with ``y = act(x @ w_in.T + b_in) @ w_out.T``: the FFN half of
     a block of width 128 whose hidden layer is 128 wide too."""
     if (x.numel() // NARROW < NARROW_MIN_TOKENS
-            or not _residual_ok(x, resid, bias, valid_len, norm, (w_in, w_out)) or b_in is None
-            or b_in.shape != (NARROW,) or not _usable(x, b_in)):
+            or not _residual_ok(allowed, x, resid, (w_in, w_out), (b_in, bias), valid_len, norm)):
         return None
     out, ln = torch.empty_like(resid), torch.empty_like(resid)
     code = _lib.lib().tj_narrow_ffn_norm(
-        x.data_ptr(), w_in.data_ptr(), b_in.data_ptr(), {"gelu": 1, "relu": 2}[act], w_out.data_ptr(),
+        x.data_ptr(), w_in.data_ptr(), b_in.data_ptr(), _ACT[act], w_out.data_ptr(),
         bias.data_ptr(), resid.data_ptr(), out.data_ptr(), x.numel() // NARROW, x.shape[1],
         None if valid_len is None else valid_len.data_ptr(), mode, norm.weight.data_ptr(), norm.bias.data_ptr(),
         ln.data_ptr(), float(norm.eps), int(bool(zero_padded_norm)), _stream_ptr(x.device))

@@ -20,7 +20,7 @@ import torch.nn.functional as F
 
 from .kernels.attention import scaled_dot_product_attention
 from .kernels.elementwise import NORM_WIDTHS
-from .kernels.linear import ffn_norm, projections, residual_norm
+from .kernels.linear import ffn_norm, projections, residual_norm, split_products_allowed
 
 
 ACTIVATIONS = ("gelu", "relu")
@@ -114,12 +114,13 @@ def fp16_weight(owner: nn.Module, key: str, weight: torch.Tensor) -> torch.Tenso
 
 
 def project(x: torch.Tensor, weight: torch.Tensor, owner: nn.Module, key: str,
-            out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """Bias-free ``x @ weight.T``. A float32 ``x`` runs the float32 GEMM; a
-    float16 ``x`` runs on fp16 operands (the weight's cached fp16 copy) with
-    fp32 accumulation, its result in ``out_dtype`` (default float16)."""
+            out_dtype: Optional[torch.dtype] = None, allowed: Optional[bool] = None) -> torch.Tensor:
+    """Bias-free ``x @ weight.T``. A float32 ``x`` runs the float32 GEMM
+    (``allowed``: what :func:`split_products_allowed` says, if the caller
+    asked); a float16 ``x`` runs on fp16 operands (the weight's cached fp16
+    copy) with fp32 accumulation, its result in ``out_dtype`` (default float16)."""
     if x.dtype != torch.float16:
-        own = projections(x, (weight,))
+        own = projections(x, (weight,), allowed=allowed)
         return _linear_f32(x, weight) if own is None else own[0]
     w16 = fp16_weight(owner, key, weight)
     if out_dtype in (None, torch.float16):
@@ -174,12 +175,13 @@ class HipSelfAttention(nn.Module):
     def project_qkv_folded(self, x: torch.Tensor):
         """Bias-free q, k, v head views (fp16 for an fp16 ``x``) and the q / v
         biases the kernel adds (a key bias never changes the attention output)."""
-        own = projections(x, (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight))
+        allowed = x.dtype == torch.float32 and split_products_allowed()
+        own = projections(x, (self.q_proj.weight, self.k_proj.weight, self.v_proj.weight), allowed=allowed)
         if own is not None:  # one launch
             return (*map(self.heads_view, own), self.q_proj.bias, self.v_proj.bias)
-        return (self.heads_view(project(x, self.q_proj.weight, self.q_proj, "weight")),
-                self.heads_view(project(x, self.k_proj.weight, self.k_proj, "weight")),
-                self.heads_view(project(x, self.v_proj.weight, self.v_proj, "weight")),
+        return (self.heads_view(project(x, self.q_proj.weight, self.q_proj, "weight", allowed=allowed)),
+                self.heads_view(project(x, self.k_proj.weight, self.k_proj, "weight", allowed=allowed)),
+                self.heads_view(project(x, self.v_proj.weight, self.v_proj, "weight", allowed=allowed)),
                 self.q_proj.bias, self.v_proj.bias)
 
     def attend(self, q, k, v, valid_len, causal):
@@ -257,9 +259,9 @@ class EncoderBlock(nn.Module):
                 and all(type(n) is nn.LayerNorm and n.elementwise_affine and n.bias is not None
                         and n.weight.dtype == torch.float32 for n in (self.norm1, self.norm2)))
 
-    def _hidden(self, a, act):
+    def _hidden(self, a, act, allowed):
         """The FFN's fp32 hidden activations, ``act(ffn_in(a))``."""
-        own = projections(a, (self.ffn_in.weight,), self.ffn_in.bias, self.activation)
+        own = projections(a, (self.ffn_in.weight,), self.ffn_in.bias, self.activation, allowed)
         if own is not None:
             return own[0]
         return _must(act(_linear_f32(a, self.ffn_in.weight), self.ffn_in.bias))
@@ -274,12 +276,12 @@ class EncoderBlock(nn.Module):
         from .kernels.elementwise import MODE_ZERO_OUT, MODE_ZERO_Y, bias_gelu, bias_relu, bias_residual
 
         act = bias_gelu if self.activation == "gelu" else bias_relu
-        attn = self.attention
+        attn, allowed = self.attention, split_products_allowed()
         ctx = attn.context(self.norm1(x), valid_token_mask, causal, valid_len)
-        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight")
+        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", allowed=allowed)
         x = _must(bias_residual(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, out=y))
-        h = self._hidden(self.norm2(x), act)
-        y = project(h, self.ffn_out.weight, self.ffn_out, "weight")
+        h = self._hidden(self.norm2(x), act, allowed)
+        y = project(h, self.ffn_out.weight, self.ffn_out, "weight", allowed=allowed)
         return _must(bias_residual(x, y, self.ffn_out.bias, valid_len, MODE_ZERO_OUT, out=y))
 
     def _forward_fused_post(self, x, valid_token_mask, causal, valid_len):
@@ -289,15 +291,15 @@ class EncoderBlock(nn.Module):
         from .kernels.elementwise import MODE_PLAIN, MODE_ZERO_Y, bias_gelu, bias_relu, bias_residual_layernorm
 
         act = bias_gelu if self.activation == "gelu" else bias_relu
-        attn = self.attention
+        attn, allowed = self.attention, split_products_allowed()
         ctx = attn.context(x, valid_token_mask, causal, valid_len)
-        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight")
+        y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", allowed=allowed)
         del ctx
         _, x = _must(bias_residual_layernorm(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, self.norm1,
                                              keep_sum=False))
         del y
-        h = self._hidden(x, act)
-        y = project(h, self.ffn_out.weight, self.ffn_out, "weight")
+        h = self._hidden(x, act, allowed)
+        y = project(h, self.ffn_out.weight, self.ffn_out, "weight", allowed=allowed)
         del h
         _, x = _must(bias_residual_layernorm(x, y, self.ffn_out.bias, valid_len, MODE_PLAIN, self.norm2,
                                              zero_padded_norm=valid_token_mask is not None, keep_sum=False))
@@ -329,7 +331,7 @@ class EncoderBlock(nn.Module):
         only the final norm, the model's output, stays fp32."""
         from .kernels.elementwise import MODE_ZERO_OUT, MODE_ZERO_Y, bias_gelu, bias_relu, bias_residual_layernorm
 
-        attn = self.attention
+        attn, allowed = self.attention, not fp16_operands and split_products_allowed()
         f32, f16 = torch.float32, torch.float16
         x, a = state
         state.clear()
@@ -339,19 +341,20 @@ class EncoderBlock(nn.Module):
         del a
         # Layers of width 128: a projection and the passes after it in one.
         own = None if fp16_operands else residual_norm(ctx, attn.out_proj.weight, attn.out_proj.bias, x, valid_len,
-                                                       MODE_ZERO_Y, self.norm2)
+                                                       MODE_ZERO_Y, self.norm2, allowed=allowed)
         if own is not None:
             del ctx
             x, a = own
         else:
-            y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", f32)
+            y = project(ctx, attn.out_proj.weight, attn.out_proj, "weight", f32, allowed)
             del ctx
             x, a = _must(bias_residual_layernorm(x, y, attn.out_proj.bias, valid_len, MODE_ZERO_Y, self.norm2, out=y,
                                                  norm_dtype=f16 if fp16_operands else f32))
             del y
         own = None if fp16_operands else ffn_norm(a, self.ffn_in.weight, self.ffn_in.bias, self.activation,
                                                   self.ffn_out.weight, self.ffn_out.bias, x, valid_len, MODE_ZERO_OUT,
-                                                  next_norm, zero_padded_norm=last and valid_token_mask is not None)
+                                                  next_norm, zero_padded_norm=last and valid_token_mask is not None,
+                                                  allowed=allowed)
         if own is not None:
             return own
         act = bias_gelu if self.activation == "gelu" else bias_relu
@@ -360,9 +363,9 @@ class EncoderBlock(nn.Module):
             # the activation straight into the fp16 operand of the next GEMM
             h = _must(act(h, self.ffn_in.bias, out_f16=True))
         else:
-            h = self._hidden(a, act)
+            h = self._hidden(a, act, allowed)
         del a
-        y = project(h, self.ffn_out.weight, self.ffn_out, "weight", f32)
+        y = project(h, self.ffn_out.weight, self.ffn_out, "weight", f32, allowed)
         del h
         return _must(bias_residual_layernorm(x, y, self.ffn_out.bias, valid_len, MODE_ZERO_OUT, next_norm, out=y,
                                              zero_padded_norm=last and valid_token_mask is not None,

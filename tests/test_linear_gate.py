@@ -17,11 +17,11 @@ _PROBE = """
 import sys, types, torch
 from techjam_amd.kernels.linear import _usable
 x = types.SimpleNamespace(is_cuda=True, dtype=torch.float32, device=torch.device("cuda", 0),
-                          is_contiguous=lambda: True, data_ptr=lambda: 0)
+                          get_device=lambda: 0, is_contiguous=lambda: True, data_ptr=lambda: 0)
 mm = torch.backends.cuda.matmul
 exec(sys.argv[1])
 with torch.no_grad():
-    print(_usable(x))
+    print(bool(_usable(None, x)))
 """
 
 
@@ -49,7 +49,7 @@ def test_a_bias_of_another_size_stays_off_the_kernel(monkeypatch, size):
     """The kernel reads as many bias values as the weight has rows."""
     from techjam_amd.kernels import linear
 
-    monkeypatch.setattr(linear, "_usable", lambda *t: True)
+    monkeypatch.setattr(linear, "_usable", lambda *t: [0] * len(t))
     monkeypatch.setattr(linear._lib, "lib", lambda: pytest.fail("the kernel would be called"))
     x, w = torch.zeros(4, 128), torch.zeros(64, 128)
     assert linear.projections(x, (w,), torch.zeros(size), "gelu") is None
