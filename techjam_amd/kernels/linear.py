@@ -21,18 +21,25 @@ from .attention import _stream_ptr
 #: Width of the layers the one-pass kernels take.
 NARROW = 128
 #: Multiply-adds up to which the small-tile kernel is used, and its depth (at
-#: K = 1024 and 256 x 256 the library takes 9.5 us, this 10.2). One product, us by the library / here, replayed as graphs: 32 x 256 x
-#: 256 11.0 / 4.4, 256 x 256 x 256 26.0 / 4.5, 256 x 512 x 512 7.5 / 6.4, 1200
-#: x 128 x 512 7.5 / 6.5; past the line 1200 x 512 x 512 11.2 / 17.2.
+#: K = 1024 and 256 x 256 the library takes 9.5 us, this 10.2). One product, us
+#: by the library / here, replayed as graphs: 32 x 256 x 256 11.0 / 4.4, 256 x
+#: 256 x 256 26.0 / 4.5, 256 x 512 x 512 7.5 / 6.4, 1200 x 128 x 512 7.5 / 6.5;
+#: past the line 1200 x 512 x 512 11.2 / 17.2. Called one after another, a
+#: lone product is bound by its call, 19.2 us by the library and 8.7 here, also
+#: where its kernel alone is behind: 4 x 1024 x 256 3.8 / 4.1, 16 x 512 x 512
+#: 4.5 / 6.0, 8192 x 128 x 64 5.1 / 6.1, and at width 128 from 4098 tokens (5.8
+#: / 7.7) to 24 576 (9.3 / 9.5). A replayed forward gives up to 2 us there.
 ROWS_MAX_WORK = 1 << 26
 ROWS_MAX_K = 512
 #: Tokens from which the one-pass kernels beat a product and the passes after
-#: it, and up to which the shorter one does (us, library + passes / here:
-#: residual + norm 16 384 tokens 16.4 / 16.4, 65 536 38 / 31, 262 144 146 / 155;
-#: FFN 30 / 38, 66 / 41, 249 / 205): below, one tile's latency is all there is.
+#: it, and up to which the shorter one does (us, library + passes / here,
+#: replayed: residual + norm 16 384 tokens 17.1 / 17.1, 24 576 21.4 / 18.2,
+#: 98 304 57 / 45, 122 880 72 / 55, 131 072 72 / 75, 262 144 151 / 161; FFN
+#: 30.7 / 30.7, 34 / 32, 95 / 61, 125 / 78 at 131 072, 259 / 166): below, one
+#: tile's latency is all there is; above, the sum in a buffer of its own takes
+#: the four tensors past the memory-side cache.
 NARROW_MIN_TOKENS = 24576
-NARROW_RESIDUAL_MAX_TOKENS = 131072
-
+NARROW_RESIDUAL_MAX_TOKENS = 122880
 
 _ACT = {None: 0, "gelu": 1, "relu": 2}
 _NONE = (None, None, None)

@@ -53,3 +53,15 @@ def test_a_bias_of_another_size_stays_off_the_kernel(monkeypatch, size):
     monkeypatch.setattr(linear._lib, "lib", lambda: pytest.fail("the kernel would be called"))
     x, w = torch.zeros(4, 128), torch.zeros(64, 128)
     assert linear.projections(x, (w,), torch.zeros(size), "gelu") is None
+
+
+@pytest.mark.parametrize("tokens,taken", [(24575, False), (24576, True), (122880, True), (131072, False)])
+def test_tokens_of_the_one_pass_residual(monkeypatch, tokens, taken):
+    """At 131 072 tokens and more the library's product and one pass are faster."""
+    from techjam_amd.kernels import linear
+
+    asked = []
+    monkeypatch.setattr(linear, "_residual_ok", lambda *a: asked.append(a))
+    x, w, b = torch.empty(1, tokens, 128, device="meta"), torch.zeros(128, 128), torch.zeros(128)
+    assert linear.residual_norm(x, w, b, x, None, 0, torch.nn.LayerNorm(128)) is None
+    assert bool(asked) == taken
