@@ -38,8 +38,9 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 // Exact GELU, x Phi(x) = max(x, 0) - |x| erfc(|x| / sqrt 2) / 2, with erfc(|x| /
 // sqrt 2) = 2^(|x| P(|x|)) and P the weighted minimax polynomial of degree 7
-// over |x| <= 5.9 (error of the erfc 1.6e-8; past that the exponent keeps
-// falling and the term is below 2e-8 |x|). One fused multiply-add ends it, so
+// over |x| <= 5.9, fitted to erfc on Chebyshev nodes by iteratively reweighted
+// least squares (Lawson's method; error of the erfc 1.6e-8; past that the
+// exponent keeps falling and the term is below 2e-8 |x|). One fused multiply-add ends it, so
 // there is no cancellation on the negative side: against 64 bits 3.2e-8,
 // 3.1e-8 and 2.9e-8 (2-norm, relative) for x ~ N(0, std^2) of std 0.05, 0.58
 // and 1, where 0.5 x (1 + erff(x / sqrt 2)) has 3.7e-8, 3.9e-8 and 3.7e-8. 14

@@ -4,9 +4,11 @@ Same module tree, parameter names and construction order as the reference
 model (``torch_transformer_benchmark.py:29-172``), so the harness's strict
 ``load_state_dict`` works unchanged and a seeded construction gives the same
 weights. Only the attention module differs: ``HipSelfAttention`` projects with
-hipBLASLt GEMMs (``Linear``, an ``nn.Linear`` whose bias add stays outside the
-GEMM when the fast float32 matmul mode is on) and calls the gfx950 attention
-kernel through the C ABI instead of materialising a score tensor.
+``Linear`` (an ``nn.Linear`` whose bias add stays outside the GEMM when the
+fast float32 matmul mode is on) and calls the gfx950 attention kernel through
+the C ABI instead of materialising a score tensor. Without gradients the
+projections run bias-free, small and 128-wide ones on the kernels of
+``kernels/linear.py``, the rest on the BLAS library (hipBLASLt by default).
 """
 
 from __future__ import annotations
